@@ -177,6 +177,23 @@ int vmoe_router_logits(const uint16_t* x, int64_t ldx, int64_t num_tokens, int64
                        const uint16_t* weight, int64_t ldw, int32_t num_experts,
                        uint16_t* logits, int64_t ld_logits, vmoe_stream_t stream);
 
+/* Backward of that linear layer from grad_logits [T, E] (contiguous):
+ *   grad_weight[e, n] = bf16(sum_t grad_logits[t, e] x[t, n])
+ *   grad_x[t, n] = bf16(sum_e grad_logits[t, e] weight[e, n]), with accumulate
+ *     != 0 added to the old grad_x[t, n] and rounded again
+ * with fp32 sums; either output may be NULL. grad_weight's sum over the tokens
+ * is cut into chunks whose fp32 sums go through `workspace`
+ * (vmoe_router_linear_bwd_workspace_bytes, possibly 0; no initial value) and
+ * are added in chunk order. Supports E % 8 == 0, E <= 128, hidden % 8 == 0 and
+ * 16-byte aligned rows (grad_weight: 8-byte); num_tokens must be positive. */
+size_t vmoe_router_linear_bwd_workspace_bytes(int64_t num_tokens, int64_t hidden,
+                                              int32_t num_experts);
+int vmoe_router_linear_bwd(const uint16_t* grad_logits, const uint16_t* x, int64_t ldx,
+                           const uint16_t* weight, int64_t ldw, int64_t num_tokens,
+                           int64_t hidden, int32_t num_experts, uint16_t* grad_x, int64_t ldgx,
+                           int32_t accumulate, uint16_t* grad_weight, int64_t ldgw,
+                           void* workspace, size_t workspace_bytes, vmoe_stream_t stream);
+
 size_t vmoe_router_partial_floats(int64_t num_tokens, int32_t num_experts);
 int vmoe_router_topk(const uint16_t* logits, int64_t ld_logits, int64_t num_tokens,
                      int32_t num_experts, int32_t top_k, int32_t normalize, uint16_t* weights,

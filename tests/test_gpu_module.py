@@ -831,3 +831,40 @@ def test_forward_without_autograd_same_bits(mode, device):
     assert bits_equal(out, out_g.detach()) and bits_equal(f_i, f_g)
     for key in aux:
         assert bits_equal(aux[key], aux_g[key].detach()), key
+
+
+@pytest.mark.parametrize("weight_grad", [False, True])
+@pytest.mark.parametrize("freeze", ["none", "x", "router", "experts"])
+def test_router_in_node_gradients(weight_grad, freeze, device):
+    """The layer with its router Linear inside the autograd node against the
+    same layer whose router has a (do-nothing) forward hook and therefore
+    keeps its own linear node: outputs, losses and every gradient bit for bit
+    (the input's is a rounded product, then a rounded sum, on both)."""
+    torch.manual_seed(3)
+    cfg = TritonMoEConfig(n_embd=136, expert_sizes=[(4, 128), (12, 64)], num_active_experts=3,
+                          routing_weight_grad=weight_grad)
+    m = TritonMoEMLP(cfg).to(device).to(torch.bfloat16)
+    x = torch.randn(2, 331, 136, device=device).to(torch.bfloat16)
+    g = torch.randn(2, 331, 136, device=device).to(torch.bfloat16)
+    m.router.weight.requires_grad_(freeze != "router")
+    for p in (m.w1, m.w2):
+        p.requires_grad_(freeze != "experts")
+
+    def step():
+        xi = x.clone().requires_grad_(freeze != "x")
+        for p in m.parameters():
+            p.grad = None
+        out, aux, f_i = m(xi)
+        names = {type(f[0]).__name__ for f in out.grad_fn.next_functions if f[0] is not None}
+        loss = (out * g).sum() + 10 * aux["router_z_loss"] + 10 * aux["load_balance_loss"]
+        loss.backward()
+        return (names, out.detach(), aux["router_z_loss"].detach(), f_i, m.w1.grad, m.w2.grad,
+                xi.grad, m.router.weight.grad)
+
+    a = step()
+    h = m.router.register_forward_hook(lambda mod, inp, out: None)
+    b = step()
+    h.remove()
+    assert a[0] != b[0] or freeze in ("router", "x")  # the hooked router has a node of its own
+    for u, v in zip(a[1:], b[1:]):
+        assert (u is None) == (v is None) and (u is None or torch.equal(u, v))

@@ -23,7 +23,7 @@ from oracle import eager
 from triton_moe import TritonMoEConfig, TritonMoEMLP
 from triton_moe.kernels.router import RouterLinear, load_balance_coef, router_topk
 
-from _util import LOOSE, assert_close_norm, bits_equal, make_problem
+from _util import LOOSE, TIGHT, assert_close_norm, bits_equal, make_problem
 
 pytestmark = pytest.mark.gpu
 
@@ -348,3 +348,62 @@ def test_router_topk_hist_routes_like_two_launches(name, device):
     # sums of T terms, f_i a function of the counts alone
     for x, y, what, rtol in zip(la, lh, ("z", "lb", "cl", "f_i"), (2.0 ** -7, 1e-5, 1e-5, 0)):
         assert torch.allclose(x.float(), y.float(), rtol=rtol, atol=0), f"{name}: aux {what}"
+
+
+@pytest.mark.parametrize("T,d,E", [(1, 128, 8), (63, 8, 8), (129, 264, 24), (700, 136, 72),
+                                   (4101, 1024, 64), (3000, 2048, 128), (257, 768, 96)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_router_linear_bwd(T, d, E, accumulate, device):
+    """vmoe_router_linear_bwd against the fp64 products at the edges of its
+    tiles (64- and 128-token steps, 128 columns, 32-expert blocks, one chunk
+    and many): one bf16 rounding of a fp32 sum, whose own error is at most
+    T (E) additions of 2^-24 of the summed magnitudes. Column slices and a
+    token row broadcast to all (stride 0) are read in place."""
+    from triton_moe import _lib
+
+    g = torch.Generator().manual_seed(T + d + E)
+    gl = torch.randn(T, E, generator=g).to(torch.bfloat16)
+    w = (torch.randn(E, d, generator=g) * 0.05).to(torch.bfloat16)
+    x = torch.randn(T, d + 8, generator=g).to(torch.bfloat16)[:, 8:]
+    gx0 = torch.randn(T, d, generator=g).to(torch.bfloat16)
+    L = _lib.lib()
+    n = L.vmoe_router_linear_bwd_workspace_bytes(T, d, E)
+    ws = torch.empty(max(n, 16), dtype=torch.uint8, device=device)
+    gld, wd = gl.to(device), w.to(device)
+    for xs in (x, x[:1].expand(T, d)):
+        xd = xs.to(device) if xs.stride(0) else xs[:1].to(device).expand(T, d)
+        if xs.stride(0):  # a slice of wider rows, as given
+            xd = torch.empty(T, d + 8, dtype=torch.bfloat16, device=device)[:, 8:].copy_(xs)
+        gx = gx0.to(device)
+        gw = torch.full((E, d), float("nan"), dtype=torch.bfloat16, device=device)
+        _lib.call("vmoe_router_linear_bwd", gld.data_ptr(), xd.data_ptr(), xd.stride(0),
+                  wd.data_ptr(), d, T, d, E, gx.data_ptr(), d, int(accumulate), gw.data_ptr(), d,
+                  ws.data_ptr(), n, _lib.stream(device))
+        for got, a, b, old in ((gw, gl.t(), xs, None), (gx, gl, w, gx0 if accumulate else None)):
+            a, b = a.double(), b.double()
+            ref, mag = a @ b, a.abs() @ b.abs()
+            bound = ref.abs() * 2.0 ** -8 + mag * (a.shape[1] * 2.0 ** -24)
+            if old is not None:  # the rounded product, then the rounded sum
+                ref = ref + old.double()
+                bound = bound * (1 + 2.0 ** -8) + ref.abs() * 2.0 ** -8
+            assert bool(((got.double().cpu() - ref).abs() <= bound).all())
+
+
+def test_router_linear_differentiable_twice(device):
+    """The router Linear's backward kernel leaves double backward, batched
+    gradients, forward mode and torch.func on the linear layer's operators."""
+    g = torch.Generator().manual_seed(1)
+    lin = RouterLinear(64, 16, bias=False).to(device).to(torch.bfloat16)
+    x = torch.randn(40, 64, generator=g).to(torch.bfloat16).to(device).requires_grad_(True)
+    v = torch.randn(3, 40, 16, generator=g).to(torch.bfloat16).to(device)
+    ref = torch.autograd.grad(F.linear(x, lin.weight), x, v[0])[0]
+    assert_close_norm(torch.autograd.grad(lin(x), x, v[0])[0], ref.float().cpu(), TIGHT, "gx")
+    gb, = torch.autograd.grad(lin(x), x, v, is_grads_batched=True)
+    assert gb.shape == (3, 40, 64) and torch.allclose(gb[0].float(), ref.float(), atol=1e-1)
+    gx, = torch.autograd.grad(lin(x).square().sum(), x, create_graph=True)
+    gw, = torch.autograd.grad(gx.sum(), lin.weight)
+    assert gw.shape == lin.weight.shape and bool(gw.isfinite().all())
+    _, jv = torch.func.jvp(lin, (x.detach(),), (x.detach(),))
+    assert torch.allclose(jv.float(), lin(x).detach().float(), atol=1e-1)
+    per = torch.func.vmap(torch.func.grad(lambda t: lin(t[None]).float().sum()))(x.detach())
+    assert per.shape == x.shape

@@ -91,6 +91,9 @@ _SIGNATURES = {
     "vmoe_gemm_f32_down_bwd_dw": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i32,
                                   _i64, _i64, _i64, _vp],
     "vmoe_router_logits": [_vp, _i64, _i64, _i64, _vp, _i64, _i32, _vp, _i64, _vp],
+    "vmoe_router_linear_bwd_workspace_bytes": [_i64, _i64, _i32],
+    "vmoe_router_linear_bwd": [_vp, _vp, _i64, _vp, _i64, _i64, _i64, _i32, _vp, _i64, _i32, _vp,
+                               _i64, _vp, ctypes.c_size_t, _vp],
     "vmoe_router_partial_floats": [_i64, _i32],
     "vmoe_router_topk": [_vp, _i64, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp,
                          ctypes.c_size_t, _vp, _vp],
@@ -124,6 +127,7 @@ _RESTYPES = {
     "vmoe_gemm_dw_workspace_bytes": ctypes.c_size_t,
     "vmoe_gemm_dw_workspace_zero_bytes": ctypes.c_size_t,
     "vmoe_router_partial_floats": ctypes.c_size_t,
+    "vmoe_router_linear_bwd_workspace_bytes": ctypes.c_size_t,
 }
 
 # Status codes (include/vmoe.h).

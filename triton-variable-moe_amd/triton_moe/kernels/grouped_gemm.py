@@ -24,11 +24,13 @@ import ctypes
 from dataclasses import dataclass
 
 import torch
+import torch.nn.functional as F
 from torch.amp import custom_bwd, custom_fwd
 from torch.autograd.function import once_differentiable
 
 from .. import _lib
 from .gather import row_maps
+from .router import router_bwd
 
 _ACTIVATIONS = {"none": _lib.ACT_NONE, "relu_squared": _lib.ACT_RELU_SQUARED}
 
@@ -1145,93 +1147,129 @@ class MoELayerOp(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, logits, x_flat, w1, w2, consts):
-        widths, ewo, coef, wn, top_k, block_size, max_width, normalize, weight_grad = consts
-        T, d = x_flat.shape
-        E = widths.shape[0]
-        dev = x_flat.device
-        x_flat = _bf16(x_flat, "TritonMoEMLP x")
-        if not logits.is_contiguous() or logits.data_ptr() % 16:
-            logits = logits.clone(memory_format=torch.contiguous_format)
-        plan = _moe_plan(T, E, top_k, block_size, d, max_width, dev)
-        saved = torch.empty(plan[0], dtype=torch.uint8, device=dev)
-        scratch = torch.empty(plan[1], dtype=torch.uint8, device=dev)
-        out = torch.empty(T, d, dtype=torch.bfloat16, device=dev)
-        z = torch.empty((), dtype=torch.bfloat16, device=dev)
-        losses = torch.empty(2, dtype=torch.float32, device=dev)
-        f_i = torch.empty(E, dtype=torch.bfloat16, device=dev)
-        if T == 0:
-            z.zero_(), losses.zero_(), f_i.zero_()
-        st = plan[7](logits.data_ptr(), T, E, top_k, int(bool(normalize)), block_size,
-                     x_flat.data_ptr(), x_flat.stride(0), w1.data_ptr(), w1.stride(0),
-                     w2.data_ptr(), w2.stride(0), ewo.data_ptr(), widths.data_ptr(), d, max_width,
-                     coef.data_ptr(), wn.data_ptr(), saved.data_ptr(), scratch.data_ptr(),
-                     out.data_ptr(), d, z.data_ptr(), losses.data_ptr(), f_i.data_ptr(),
-                     _lib.stream(dev))
-        if st != _lib.OK:
-            _lib.check(st, "vmoe_moe_forward")
-        ctx.save_for_backward(logits, x_flat, w1, w2, saved)
-        # the module's constant tables (buffers, never written in place)
-        ctx.consts = consts
-        ctx.dims = (T, E, d, int(bool(normalize)))
-        ctx.mark_non_differentiable(f_i)
-        # unused outputs arrive as None (not zeros), so a loss that leaves out
-        # the auxiliary losses gives the router no gradient, as in the reference
-        ctx.set_materialize_grads(False)
-        return out, z, losses[0], losses[1], f_i
+        return _moe_forward(ctx, logits, x_flat, w1, w2, None, consts)
 
     @staticmethod
     @once_differentiable
     def backward(ctx, grad_out, g_z, g_lb, g_cl, _g_fi):
-        logits, x_flat, w1, w2, saved = ctx.saved_tensors
-        widths, ewo, coef, wn, k, b, max_width, _, weight_grad = ctx.consts
-        T, E, d, norm = ctx.dims
-        dev = logits.device
-        plan = _moe_plan(T, E, k, b, d, max_width, dev)
-
-        def scalar(g):
-            return None if g is None else g.detach().to(torch.float32).reshape(()).contiguous()
-
-        gz, glb, gcl = scalar(g_z), scalar(g_lb), scalar(g_cl)
         need = ctx.needs_input_grad
-        want_x = grad_out is not None and (need[1] or need[2] or need[3])
-        want_logits = need[0] and (
-            gz is not None or glb is not None or gcl is not None or (weight_grad and want_x))
-        grad_x = grad_w1 = grad_w2 = grad_logits = None
-        g = gs = None
-        ldg = 0
-        if want_x:
-            if (grad_out.dtype == torch.bfloat16 and T > 0 and grad_out.stride(0) == 0 and
-                    grad_out.stride(1) == 0):
-                g, ldg, gs = plan[6], 0, grad_out  # c * out.sum(): ones times c
-            else:
-                (g, ldg), gs = _token_source(grad_out), None
-            grad_x = torch.empty(T, d, dtype=torch.bfloat16, device=dev)
-            # no tokens: the library writes nothing, the weight gradients are zero
-            grad_w1 = torch.empty_like(w1) if T > 0 else torch.zeros_like(w1)
-            grad_w2 = torch.empty_like(w2) if T > 0 else torch.zeros_like(w2)
-        if want_logits:
-            grad_logits = torch.empty(T, E, dtype=torch.bfloat16, device=dev)
-        if not want_x and not want_logits:
-            return None, None, None, None, None
-        scratch = torch.empty(plan[2], dtype=torch.uint8, device=dev)
-        main = _lib.stream(dev)
-        use_side = BACKWARD_SIDE_STREAM if BACKWARD_SIDE_STREAM is not None else plan[5]
-        side = _side_stream(dev).cuda_stream if use_side else None
-        ws_stream = side if side is not None else main
-        ws = _DW_WORKSPACES.get((dev.index, ws_stream))
-        if ws is None or ws.numel() < plan[4]:
-            ws = _dw_workspace_bytes(E, d, max_width, plan[3], dev, ws_stream)
-        ptr = _lib.ptr
-        st = plan[8](saved.data_ptr(), logits.data_ptr(), T, E, k, norm, b,
-                     x_flat.data_ptr(), x_flat.stride(0), w1.data_ptr(), w1.stride(0),
-                     w2.data_ptr(), w2.stride(0), ewo.data_ptr(), widths.data_ptr(), d, max_width,
-                     coef.data_ptr(), wn.data_ptr(), ptr(g), ldg, ptr(gs), ptr(gz), ptr(glb),
-                     ptr(gcl), int(bool(weight_grad)), ptr(grad_x), d, ptr(grad_w1), w1.stride(0),
-                     ptr(grad_w2), w2.stride(0), ptr(grad_logits), scratch.data_ptr(),
-                     ws.data_ptr(), ws.numel(), main, side)
-        if st != _lib.OK:
-            _lib.check(st, "vmoe_moe_backward")
+        grad_logits, grad_x, grad_w1, grad_w2 = _moe_backward(
+            ctx, grad_out, g_z, g_lb, g_cl, need[0], need[1] or need[2] or need[3])
         return grad_logits, grad_x, grad_w1, grad_w2, None
+
+
+class MoERouterLayerOp(torch.autograd.Function):
+    """MoELayerOp with the router Linear inside the node: forward(x_flat, wr,
+    w1, w2, consts), the logits being F.linear(x_flat, wr), the bits of the
+    router module's own forward. The backward forms both router gradients in
+    one launch (vmoe_router_linear_bwd; the token gradient is added to the
+    expert path's in place), where autograd's linear node took two GEMM
+    launches and an add over [T, hidden]."""
+
+    @staticmethod
+    def forward(ctx, x_flat, wr, w1, w2, consts):
+        return _moe_forward(ctx, F.linear(x_flat, wr), x_flat, w1, w2, wr, consts)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_out, g_z, g_lb, g_cl, _g_fi):
+        need_x, need_wr, need_w1, need_w2, _ = ctx.needs_input_grad
+        grad_logits, grad_x, grad_w1, grad_w2 = _moe_backward(
+            ctx, grad_out, g_z, g_lb, g_cl, need_x or need_wr, need_x or need_w1 or need_w2)
+        grad_wr = None
+        if grad_logits is not None:
+            grad_x, grad_wr = router_bwd(grad_logits, ctx.saved_tensors[1], ctx.saved_tensors[5],
+                                         need_x, need_wr, grad_x)
+        return grad_x, grad_wr, grad_w1, grad_w2, None
+
+
+def _moe_forward(ctx, logits, x_flat, w1, w2, wr, consts):
+    widths, ewo, coef, wn, top_k, block_size, max_width, normalize, weight_grad = consts
+    T, d = x_flat.shape
+    E = widths.shape[0]
+    dev = x_flat.device
+    x_flat = _bf16(x_flat, "TritonMoEMLP x")
+    if not logits.is_contiguous() or logits.data_ptr() % 16:
+        logits = logits.clone(memory_format=torch.contiguous_format)
+    plan = _moe_plan(T, E, top_k, block_size, d, max_width, dev)
+    saved = torch.empty(plan[0], dtype=torch.uint8, device=dev)
+    scratch = torch.empty(plan[1], dtype=torch.uint8, device=dev)
+    out = torch.empty(T, d, dtype=torch.bfloat16, device=dev)
+    z = torch.empty((), dtype=torch.bfloat16, device=dev)
+    losses = torch.empty(2, dtype=torch.float32, device=dev)
+    f_i = torch.empty(E, dtype=torch.bfloat16, device=dev)
+    if T == 0:
+        z.zero_(), losses.zero_(), f_i.zero_()
+    st = plan[7](logits.data_ptr(), T, E, top_k, int(bool(normalize)), block_size,
+                 x_flat.data_ptr(), x_flat.stride(0), w1.data_ptr(), w1.stride(0),
+                 w2.data_ptr(), w2.stride(0), ewo.data_ptr(), widths.data_ptr(), d, max_width,
+                 coef.data_ptr(), wn.data_ptr(), saved.data_ptr(), scratch.data_ptr(),
+                 out.data_ptr(), d, z.data_ptr(), losses.data_ptr(), f_i.data_ptr(),
+                 _lib.stream(dev))
+    if st != _lib.OK:
+        _lib.check(st, "vmoe_moe_forward")
+    ctx.save_for_backward(logits, x_flat, w1, w2, saved, *(() if wr is None else (wr,)))
+    # the module's constant tables (buffers, never written in place)
+    ctx.consts = consts
+    ctx.dims = (T, E, d, int(bool(normalize)))
+    ctx.mark_non_differentiable(f_i)
+    # unused outputs arrive as None (not zeros), so a loss that leaves out
+    # the auxiliary losses gives the router no gradient, as in the reference
+    ctx.set_materialize_grads(False)
+    return out, z, losses[0], losses[1], f_i
+
+
+def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts):
+    """(grad_logits, grad_x, grad_w1, grad_w2), None where not formed."""
+    logits, x_flat, w1, w2, saved = ctx.saved_tensors[:5]
+    widths, ewo, coef, wn, k, b, max_width, _, weight_grad = ctx.consts
+    T, E, d, norm = ctx.dims
+    dev = logits.device
+    plan = _moe_plan(T, E, k, b, d, max_width, dev)
+
+    def scalar(g):
+        return None if g is None else g.detach().to(torch.float32).reshape(()).contiguous()
+
+    gz, glb, gcl = scalar(g_z), scalar(g_lb), scalar(g_cl)
+    want_x = grad_out is not None and need_experts
+    want_logits = need_logits and (
+        gz is not None or glb is not None or gcl is not None or (weight_grad and want_x))
+    grad_x = grad_w1 = grad_w2 = grad_logits = None
+    g = gs = None
+    ldg = 0
+    if want_x:
+        if (grad_out.dtype == torch.bfloat16 and T > 0 and grad_out.stride(0) == 0 and
+                grad_out.stride(1) == 0):
+            g, ldg, gs = plan[6], 0, grad_out  # c * out.sum(): ones times c
+        else:
+            (g, ldg), gs = _token_source(grad_out), None
+        grad_x = torch.empty(T, d, dtype=torch.bfloat16, device=dev)
+        # no tokens: the library writes nothing, the weight gradients are zero
+        grad_w1 = torch.empty_like(w1) if T > 0 else torch.zeros_like(w1)
+        grad_w2 = torch.empty_like(w2) if T > 0 else torch.zeros_like(w2)
+    if want_logits:
+        grad_logits = torch.empty(T, E, dtype=torch.bfloat16, device=dev)
+    if not want_x and not want_logits:
+        return None, None, None, None
+    scratch = torch.empty(plan[2], dtype=torch.uint8, device=dev)
+    main = _lib.stream(dev)
+    use_side = BACKWARD_SIDE_STREAM if BACKWARD_SIDE_STREAM is not None else plan[5]
+    side = _side_stream(dev).cuda_stream if use_side else None
+    ws_stream = side if side is not None else main
+    ws = _DW_WORKSPACES.get((dev.index, ws_stream))
+    if ws is None or ws.numel() < plan[4]:
+        ws = _dw_workspace_bytes(E, d, max_width, plan[3], dev, ws_stream)
+    ptr = _lib.ptr
+    st = plan[8](saved.data_ptr(), logits.data_ptr(), T, E, k, norm, b,
+                 x_flat.data_ptr(), x_flat.stride(0), w1.data_ptr(), w1.stride(0),
+                 w2.data_ptr(), w2.stride(0), ewo.data_ptr(), widths.data_ptr(), d, max_width,
+                 coef.data_ptr(), wn.data_ptr(), ptr(g), ldg, ptr(gs), ptr(gz), ptr(glb),
+                 ptr(gcl), int(bool(weight_grad)), ptr(grad_x), d, ptr(grad_w1), w1.stride(0),
+                 ptr(grad_w2), w2.stride(0), ptr(grad_logits), scratch.data_ptr(),
+                 ws.data_ptr(), ws.numel(), main, side)
+    if st != _lib.OK:
+        _lib.check(st, "vmoe_moe_backward")
+    return grad_logits, grad_x, grad_w1, grad_w2
 
 
 class NoTokensOp(torch.autograd.Function):

@@ -134,6 +134,77 @@ class RouterLogitsOp(torch.autograd.Function):
         return gx, gw
 
 
+def router_bwd_supported(wr: torch.Tensor) -> bool:
+    """Router weights vmoe_router_linear_bwd takes (bf16 on the GPU, E % 8 == 0,
+    E <= 128, hidden % 8 == 0, 16-byte aligned rows)."""
+    E, d = wr.shape
+    return (wr.dtype == torch.bfloat16 and wr.is_cuda and E % 8 == 0 and E <= 128 and
+            d % 8 == 0 and wr.stride(1) == 1 and wr.stride(0) % 8 == 0 and
+            wr.stride(0) >= d and wr.data_ptr() % 16 == 0)
+
+
+def router_bwd(g: torch.Tensor, x2d: torch.Tensor, wr: torch.Tensor, need_x: bool, need_w: bool,
+               grad_x: torch.Tensor | None = None):
+    """(grad_x, grad_w) of the router Linear from contiguous logit gradients g
+    [T, E] (vmoe_router_linear_bwd); a grad_x given is added to in place."""
+    T, d = x2d.shape
+    E = wr.shape[0]
+    dev = g.device
+    add = grad_x is not None
+    if need_x and not add:
+        grad_x = torch.empty(T, d, dtype=torch.bfloat16, device=dev)
+    grad_w = torch.empty(E, d, dtype=torch.bfloat16, device=dev) if need_w else None
+    n = int(_lib.lib().vmoe_router_linear_bwd_workspace_bytes(T, d, E)) if need_w else 0
+    ws = torch.empty(n, dtype=torch.uint8, device=dev) if n else None
+    _lib.call("vmoe_router_linear_bwd", g.data_ptr(), x2d.data_ptr(), x2d.stride(0),
+              wr.data_ptr(), wr.stride(0), T, d, E, grad_x.data_ptr() if need_x else None, d,
+              int(add), _lib.ptr(grad_w), d, _lib.ptr(ws), n, _lib.stream(dev))
+    return grad_x, grad_w
+
+
+def _eager_call(*tensors: torch.Tensor) -> bool:
+    """Plain tensors outside every transform that must see torch operators
+    (tracing, torch.func, forward-mode AD, dispatch modes)."""
+    return (all((type(t) is torch.Tensor or type(t) is nn.Parameter) and
+                torch._C._has_storage(t) for t in tensors) and
+            not torch.compiler.is_compiling() and not torch.jit.is_tracing() and
+            torch._C._functorch.peek_interpreter_stack() is None and
+            torch.autograd.forward_ad._current_level < 0 and
+            torch._C._len_torch_dispatch_stack() == 0)
+
+
+class RouterLinearOp(torch.autograd.Function):
+    """F.linear(x, w) whose backward is vmoe_router_linear_bwd; a backward that
+    is itself differentiated or batched is the linear layer's two matmuls."""
+
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(x, w)
+        ctx.set_materialize_grads(False)  # unused logits give no gradient, not zeros
+        return F.linear(x, w)
+
+    @staticmethod
+    def backward(ctx, g):
+        if g is None:
+            return None, None
+        x, w = ctx.saved_tensors
+        need_x, need_w = ctx.needs_input_grad
+        if torch.is_grad_enabled() or not _eager_call(g, x, w) or g.dtype != torch.bfloat16:
+            gx = g.matmul(w) if need_x else None
+            gw = (g.reshape(-1, g.shape[-1]).t().matmul(x.reshape(-1, x.shape[-1]))
+                  if need_w else None)
+            return gx, gw
+        g = g.reshape(-1, g.shape[-1])
+        if not g.is_contiguous() or g.data_ptr() % 16:
+            g = g.clone(memory_format=torch.contiguous_format)
+        x2d = x.reshape(-1, x.shape[-1])
+        if x2d.stride(1) != 1 or x2d.stride(0) % 8 or x2d.data_ptr() % 16 or (
+                0 < x2d.stride(0) < x2d.shape[1]):
+            x2d = x2d.clone(memory_format=torch.contiguous_format)
+        gx, gw = router_bwd(g, x2d, w, need_x, need_w)
+        return None if gx is None else gx.view(x.shape), gw
+
+
 class RouterLinear(nn.Linear):
     """The router of TritonMoEMLP: nn.Linear(n_embd, num_experts, bias=False)
     (moe.py:78 of the reference) -- same parameter, initialisation, state-dict
@@ -142,7 +213,9 @@ class RouterLinear(nn.Linear):
     Its forward is nn.Linear's own (F.linear, hipBLASLt on ROCm), so the
     logits carry the same bits as the reference module's on the same GPU and
     the routing decisions downstream (top-k of their sigmoid, which the
-    router kernel reproduces bit for bit) are the reference's. With
+    router kernel reproduces bit for bit) are the reference's. The gradients of
+    the shapes vmoe_router_linear_bwd takes are formed by that kernel
+    (RouterLinearOp). With
     use_logits_kernel = True the inputs vmoe_router_logits supports go to that
     kernel instead: one bf16 rounding of the fp32 product, in its own
     summation order, which can move a logit by one bf16 step (about 0.02 %
@@ -156,6 +229,11 @@ class RouterLinear(nn.Linear):
                 router_logits_supported(x, self.weight)):
             out = RouterLogitsOp.apply(x.reshape(-1, x.shape[-1]), self.weight)
             return out.reshape(*x.shape[:-1], out.shape[-1])
+        if (torch.is_grad_enabled() and self.bias is None and _eager_call(x, self.weight) and
+                (x.requires_grad or self.weight.requires_grad) and x.is_cuda and
+                x.dtype == torch.bfloat16 and x.dim() > 1 and x.numel() > 0 and
+                not torch.is_autocast_enabled() and router_bwd_supported(self.weight)):
+            return RouterLinearOp.apply(x, self.weight)
         return F.linear(x, self.weight, self.bias)
 
 

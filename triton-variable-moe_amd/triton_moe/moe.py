@@ -25,6 +25,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from einops import rearrange
+from torch.nn.modules import module as nn_module
 
 from .kernels import (
     fused_route,
@@ -38,10 +39,11 @@ from .kernels.fused_cumsum import route_device
 from .kernels.gather import combine_rows
 from .kernels import grouped_gemm as gg
 from .kernels.grouped_gemm import (CompactRoutedMoEOp, ExpertPathOp, GemmMeta, MoELayerOp,
-                                   NoTokensOp,
+                                   MoERouterLayerOp, NoTokensOp,
                                    RoutedMoEOp, RoutedMoEOpF32, down_fwd, f32_down_fwd,
                                    f32_up_fwd, up_fwd)
-from .kernels.router import RouterAuxOp, RouterLinear, RouterWeightOp, router_topk
+from .kernels.router import (RouterAuxOp, RouterLinear, RouterWeightOp, router_bwd_supported,
+                             router_topk)
 
 
 @dataclass
@@ -288,6 +290,29 @@ class TritonMoEMLP(nn.Module):
                                            r.row_src, r.assignment_row, w, k, self.config.n_embd)
         return output_flat, r.tokens_per_expert
 
+    def _layer_consts(self, coef, wn) -> tuple:
+        """MoELayerOp's constant tables and settings."""
+        return (self.expert_widths_t, self.expert_weight_offsets_t, coef, wn,
+                self.num_active_experts, self.block_size, self.max_expert_width,
+                self.norm_topk_prob,
+                self.config.routing_weight_grad and torch.is_grad_enabled())
+
+    def _router_in_node(self, x_flat) -> bool:
+        """Whether the router Linear runs inside the layer's autograd node
+        (MoERouterLayerOp): a plain RouterLinear whose call would be F.linear
+        and nothing else (no hooks of its own or global ones, no replaced
+        forward, no autocast), on the one-node bf16 path and the shapes its
+        backward kernel takes. Anything else keeps the router's own call."""
+        r = self.router
+        if (type(r) is not RouterLinear or x_flat.shape[0] == 0 or
+                x_flat.dtype != torch.bfloat16 or self.w1.dtype != torch.bfloat16):
+            return False
+        return (gg.FUSED_EXPERT_PATH and _lib._launch_timer is None and not self._compact() and
+                r.bias is None and not r.use_logits_kernel and "forward" not in r.__dict__ and
+                not (r._forward_hooks or r._forward_pre_hooks or r._backward_hooks or
+                     r._backward_pre_hooks) and not nn_module._has_any_global_hook() and
+                not torch.is_autocast_enabled() and router_bwd_supported(r.weight))
+
     @torch.compiler.disable
     def forward(
         self, x: torch.Tensor
@@ -295,6 +320,13 @@ class TritonMoEMLP(nn.Module):
         """x [batch, seq, n_embd] -> (output [batch, seq, n_embd], aux_loss dict, f_i)."""
         batch_size, seq_len, n_embd = x.shape
         x_flat = x.reshape(batch_size * seq_len, n_embd)  # rearrange "b s d -> (b s) d"
+        if torch.is_grad_enabled() and self._router_in_node(x_flat):
+            # the router Linear too: its gradients come out of the same node
+            coef, wn = self._aux_tables(x_flat.device)
+            out, z, lb, cl, f_i = MoERouterLayerOp.apply(
+                x_flat, self.router.weight, self.w1, self.w2, self._layer_consts(coef, wn))
+            aux_loss = {"router_z_loss": z, "load_balance_loss": lb, "compute_loss": cl}
+            return out.view(batch_size, seq_len, n_embd), aux_loss, f_i.to(x.dtype)
         router_logits = self.router(x_flat)
         # (a batch without tokens always takes the one-node path, which returns
         # an empty output, zero losses and zero weight gradients)
@@ -304,11 +336,7 @@ class TritonMoEMLP(nn.Module):
             # everything after the router Linear: one node, one call each way
             coef, wn = self._aux_tables(router_logits.device)
             out, z, lb, cl, f_i = MoELayerOp.apply(
-                router_logits, x_flat, self.w1, self.w2,
-                (self.expert_widths_t, self.expert_weight_offsets_t, coef, wn,
-                 self.num_active_experts, self.block_size, self.max_expert_width,
-                 self.norm_topk_prob,
-                 self.config.routing_weight_grad and torch.is_grad_enabled()))
+                router_logits, x_flat, self.w1, self.w2, self._layer_consts(coef, wn))
             aux_loss = {"router_z_loss": z, "load_balance_loss": lb, "compute_loss": cl}
             return out.view(batch_size, seq_len, n_embd), aux_loss, f_i.to(x.dtype)
         state = router_topk(router_logits, self.num_active_experts, self.norm_topk_prob,

@@ -39,6 +39,12 @@ CASES = {
     "wide": ([300, 257], [256, 512], 256, False),
     # hidden, widths and offsets off the bf16 kernels' multiple-of-8 rule
     "unaligned": ([50, 33, 0, 17], [12, 20, 36, 5], 100, False),
+    # one off the 64-wide tiles and 32-deep k steps either way, and widths that
+    # are and are not multiples of 4 in one launch
+    "tile_edges": ([63, 64, 65, 1, 129], [63, 64, 65, 33, 31], 132, False),
+    # more experts than the tile search counts at a time
+    "many_experts": ([3 * (e % 5) for e in range(150)], [4 + 4 * (e % 3) for e in range(150)],
+                     68, False),
 }
 
 

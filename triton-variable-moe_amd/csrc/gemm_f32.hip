@@ -1,24 +1,28 @@
-// fp32 grouped GEMMs: the float32 inputs of the public grouped-GEMM API.
+// fp32 grouped GEMMs: the float32 inputs of the public grouped-GEMM API and
+// the float32 module.
 //
 // The reference's grouped-GEMM kernels take fp32 as well as bf16 operands
 // (triton_moe/kernels/grouped_gemm.py:217-1162, dtype-generic tl.dot with an
 // fp32 accumulator); its autograd tests and forward/backward benchmark run
 // them in fp32 (tests/test_grouped_gemm_backward.py:151-208). The bf16 kernels
-// of gemm.hip stage bf16 tiles for MFMA and cannot take fp32, so this file
-// holds one LDS-tiled fp32 VALU kernel for all six forms (up forward with its
-// activation, down forward, and both backward GEMMs of each). Every product
-// is an fp32 fma in k order per output, outputs are stored in fp32, and the
-// activation gradients (relu^2, SwiGLU's [dG | dU]) are formed from
-// grad/pre/up as the operand tile is loaded, as the reference's backward
-// kernels do (grouped_gemm.py:751-764, 914-927), so no launch sits between
-// the GEMMs. This is the path for fp32 callers; the bf16 module path never
-// uses it.
+// of gemm.hip stage bf16 tiles and cannot take fp32, so this file holds one
+// LDS-tiled kernel for all six forms (up forward with its activation, down
+// forward, and both backward GEMMs of each) on v_mfma_f32_32x32x2_f32: fp32
+// products and sums, nothing narrower. The activation gradients (SwiGLU's
+// [dG | dU]) are formed from grad/pre/up as the operand tile is loaded, as the
+// reference's backward kernels do (grouped_gemm.py:751-764, 914-927).
 //
-// Tiles: 64 x 64 outputs per 256-thread workgroup, 4 x 4 per thread (4
-// consecutive rows by 4 consecutive columns), k steps of 16 staged in LDS, each thread loading runs of 4 consecutive elements
-// (16-byte loads where the address is aligned and the run in range). Workgroups stride over the experts' tiles in order,
-// read from the metadata on the device (no host sync).
+// What bounds it: the fp32 matrix rate (256 flop per cycle and CU, 157 TFLOP/s
+// at 2.4 GHz; the vector pipe without packed fp32, which this build does not
+// use, has half of it: the fma kernel this replaced ran cfg-like shapes of
+// 8192 rows x 768 x 512 at 42 TFLOP/s). That rate is low enough that a 64 x 64 tile
+// per 256-thread workgroup, one 32 x 32 block per wave, needs only 16 bytes
+// per cycle and CU from L2 and 32 from LDS, so the tile is chosen small for
+// balance and occupancy: up to 8 workgroups share a CU and hide each other's
+// loads, and the widths and row counts of real experts leave little of a tile
+// empty.
 #include <algorithm>
+#include <type_traits>
 
 #include "vmoe_common.h"
 
@@ -28,9 +32,17 @@ namespace {
 enum F32Form { F_UP_FWD, F_DOWN_FWD, F_UP_DX, F_UP_DW, F_DOWN_DH, F_DOWN_DW };
 
 constexpr int kT = 64;        // tile edge
-constexpr int kBK = 16;       // k per LDS stage
+constexpr int kBK = 32;       // k per LDS stage
 constexpr int kThreads = 256;
-constexpr int kPad = kT + 4;  // LDS row length (floats)
+constexpr int kRuns = kT * kBK / 4 / kThreads;  // runs of 4 floats per thread and operand stage
+// LDS rows (floats). An operand that is contiguous along k is held as [x][k],
+// one 16-byte read giving a lane 4 consecutive k: rows of 36 floats put the 16
+// rows one phase reads on different banks. Any other is held as [k][x], one
+// 4-byte read per k: rows of 72 floats put the two rows 4 apart that the
+// halves of a wave read on different banks.
+constexpr int kRowK = kBK + 4, kRowX = kT + 8;
+constexpr int kStage = kT * kRowK > kBK * kRowX ? kT * kRowK : kBK * kRowX;
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 struct F32Args {
   // token-row operand: x (up forms), h (down forms) or grad_y (dH)
@@ -167,8 +179,8 @@ __device__ __forceinline__ float4 load_run(const float* ptr, int64_t valid) {
 }
 
 // Four elements of A from (m, k) along its contiguous dimension (k for the
-// K-contiguous forms, m otherwise); not for up dX, whose A is the
-// activation gradient (stage_elem).
+// K-contiguous forms, m otherwise); up dX only without an activation (with
+// one, its A is formed element by element).
 template <int F>
 __device__ __forceinline__ float4 f32_a_run(const F32Args& p, const F32Prob& q, int64_t m,
                                             int64_t k) {
@@ -179,6 +191,8 @@ __device__ __forceinline__ float4 f32_a_run(const F32Args& p, const F32Prob& q, 
       const float* row = token_row(p, q.t0 + m);
       return load_run(row ? row + k : nullptr, q.K - k);
     }
+    case F_UP_DX:  // the gradient itself (no activation)
+      return m < q.M ? load_run(p.g + (q.t0 + m) * p.ldg + k, q.K - k) : z;
     case F_DOWN_FWD:
     case F_DOWN_DH:
       return m < q.M ? load_run(p.a + (q.t0 + m) * p.lda + k, q.K - k) : z;
@@ -193,8 +207,7 @@ __device__ __forceinline__ float4 f32_a_run(const F32Args& p, const F32Prob& q, 
 }
 
 // Four elements of B from (k, n) along its contiguous dimension (k for up dX
-// and down dH, n otherwise); not for up dW, whose B is the activation
-// gradient (stage_elem).
+// and down dH, n otherwise); up dW only without an activation.
 template <int F>
 __device__ __forceinline__ float4 f32_b_run(const F32Args& p, const F32Prob& q, int64_t k,
                                             int64_t n, bool second) {
@@ -206,6 +219,8 @@ __device__ __forceinline__ float4 f32_b_run(const F32Args& p, const F32Prob& q, 
       return k < q.K ? load_run(p.b + (q.w0 + k) * p.ldb + n, q.N - n) : z;
     case F_UP_DX:  // W1^T
       return n < q.N ? load_run(p.b + n * p.ldb + q.w0 + k, q.K - k) : z;
+    case F_UP_DW:  // the gradient itself (no activation)
+      return k < q.K ? load_run(p.g + (q.t0 + k) * p.ldg + n, q.N - n) : z;
     case F_DOWN_DH:  // W2^T
       return n < q.N ? load_run(p.b + (q.w0 + n) * p.ldb + k, q.K - k) : z;
     default:  // F_DOWN_DW: grad_y
@@ -213,146 +228,358 @@ __device__ __forceinline__ float4 f32_b_run(const F32Args& p, const F32Prob& q, 
   }
 }
 
-// Loads a kBK x kT stage into lds[k][x] element by element, consecutive
-// lanes along the operand's contiguous dimension (the activation-gradient
-// operands, formed per element).
-template <bool KCONTIG, typename Fn>
-__device__ __forceinline__ void stage_elem(float (*lds)[kPad], Fn&& at) {
+// Runs of 4 elements of a kBK x kT operand stage: thread -> (k, x) of run i,
+// along the operand's contiguous dimension (k when KCONTIG).
+template <bool KCONTIG>
+__device__ __forceinline__ void run_at(int i, int& k, int& x) {
   const int tid = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int k, x;
-    if (KCONTIG) {
-      k = tid & (kBK - 1);
-      x = (tid >> 4) + 16 * i;
-    } else {
-      x = tid & (kT - 1);
-      k = (tid >> 6) + 4 * i;
-    }
-    lds[k][x] = at(k, x);
+  if (KCONTIG) {
+    x = (tid >> 3) + 32 * i;
+    k = (tid & 7) * 4;
+  } else {
+    x = (tid & 15) * 4;
+    k = (tid >> 4) + 16 * i;
   }
 }
 
-// Loads a kBK x kT stage into lds[k][x]: one run of 4 elements per thread
-// along the operand's contiguous dimension (k when KCONTIG, x otherwise).
 template <bool KCONTIG, typename Fn>
-__device__ __forceinline__ void stage(float (*lds)[kPad], Fn&& run) {
-  const int tid = threadIdx.x;
-  if (KCONTIG) {
-    const int x = tid >> 2, k = (tid & 3) * 4;
-    const float4 v = run(k, x);
-    lds[k][x] = v.x;
-    lds[k + 1][x] = v.y;
-    lds[k + 2][x] = v.z;
-    lds[k + 3][x] = v.w;
-  } else {
-    const int x = (tid & 15) * 4, k = tid >> 4;
-    const float4 v = run(k, x);
-    lds[k][x] = v.x;
-    lds[k][x + 1] = v.y;
-    lds[k][x + 2] = v.z;
-    lds[k][x + 3] = v.w;
+__device__ __forceinline__ void load_stage(float4 (&r)[kRuns], Fn&& run) {
+#pragma unroll
+  for (int i = 0; i < kRuns; ++i) {
+    int k, x;
+    run_at<KCONTIG>(i, k, x);
+    r[i] = run(k, x);
   }
+}
+
+template <bool KCONTIG>
+__device__ __forceinline__ void store_stage(float* lds, const float4 (&r)[kRuns]) {
+#pragma unroll
+  for (int i = 0; i < kRuns; ++i) {
+    int k, x;
+    run_at<KCONTIG>(i, k, x);
+    *reinterpret_cast<float4*>(lds + (KCONTIG ? x * kRowK + k : k * kRowX + x)) = r[i];
+  }
+}
+
+// The lane's operand values of 8 consecutive k from kk: element j is (x = x0 +
+// lane % 32, k = kk + 4 (lane / 32) + j), so MFMA j takes k = kk + j from the
+// lower and kk + 4 + j from the upper half of the wave.
+template <bool KCONTIG>
+__device__ __forceinline__ float4 frag(const float* lds, int x0, int kk) {
+  const int lane = threadIdx.x & 63;
+  const int x = x0 + (lane & 31), k = kk + 4 * (lane >> 5);
+  if (KCONTIG) return *reinterpret_cast<const float4*>(lds + x * kRowK + k);
+  const float* c = lds + k * kRowX + x;
+  return make_float4(c[0], c[kRowX], c[2 * kRowX], c[3 * kRowX]);
+}
+
+__device__ __forceinline__ void mfma4(f32x16_t& acc, const float4& a, const float4& b) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
+}
+
+// The expert and tile of item j of this workgroup's XCD: each wave counts the tiles of 64
+// experts at a time, one per lane, and scans them (a walk over the experts one
+// by one costs a dependent load per expert). XCD x takes a contiguous eighth
+// of the tiles, so the tiles that share rows or columns share an L2. Returns
+// false past the last tile.
+template <int F>
+__device__ __forceinline__ bool find_tile(const F32Args& p, int64_t j, int& expert,
+                                          int64_t& local) {
+  const int lane = threadIdx.x & 63;
+  auto tiles_of = [&](int e) -> int {
+    if (e >= p.E) return 0;
+    const F32Prob q = f32_prob<F>(p, e);
+    return (int)(cdiv64(q.M, kT) * cdiv64(q.N, kT));
+  };
+  int64_t total = 0;
+  int first = 0;  // the lane's count and its wave's inclusive scan for experts 0 .. 63
+  for (int e0 = 0; e0 < p.E; e0 += kWave) {
+    const int inc = wave_inclusive_scan(tiles_of(e0 + lane));
+    if (e0 == 0) first = inc;
+    total += __shfl(inc, kWave - 1);
+  }
+  const int64_t per = (total + 7) / 8;
+  const int64_t t = (blockIdx.x & 7) * per + j;
+  if (j >= per || t >= total) return false;
+  int64_t before = 0;
+  for (int e0 = 0; e0 < p.E; e0 += kWave) {
+    const int inc = e0 == 0 ? first : wave_inclusive_scan(tiles_of(e0 + lane));
+    const uint64_t past = ballot64(before + inc > t);
+    if (past) {
+      const int l = __builtin_ctzll(past);
+      expert = __builtin_amdgcn_readfirstlane(e0 + l);
+      local = t - before - (l > 0 ? __shfl(inc, l - 1) : 0);
+      return true;
+    }
+    before += __shfl(inc, kWave - 1);
+  }
+  return false;
+}
+
+// Operand sources of a form: the matrix its A and B come from and the leading
+// dimensions (the gradient g for up dX's A and up dW's B).
+template <int F>
+__device__ __forceinline__ const float* a_src(const F32Args& p) { return F == F_UP_DX ? p.g : p.a; }
+template <int F>
+__device__ __forceinline__ int64_t a_ld(const F32Args& p) { return F == F_UP_DX ? p.ldg : p.lda; }
+template <int F>
+__device__ __forceinline__ const float* b_src(const F32Args& p) { return F == F_UP_DW ? p.g : p.b; }
+template <int F>
+__device__ __forceinline__ int64_t b_ld(const F32Args& p) { return F == F_UP_DW ? p.ldg : p.ldb; }
+
+// Stage loads without branches: buffer loads at 32-bit offsets from the tile's
+// corner, where an offset past the resource reads zeros. `wide` (tile_wide)
+// tiles have every run of 4 floats wholly inside or outside the operand and
+// 16-byte aligned and load it at once, the others element by element. (The
+// general loads, f32_a_run and f32_b_run, test every run's alignment and every
+// element of a cut one behind branches, at 64-bit addresses; that code took
+// longer than the stage's MFMAs: 8192 rows x 768 x 512, 106 us a GEMM with it,
+// 79-90 without.)
+constexpr uint32_t kOob = 0x80000000u;
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t f32_rsrc(const float* b) {
+  const uint64_t v = reinterpret_cast<uint64_t>(b);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc(
+      reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), 0, 0x7FFFFFFF, 0x00020000);
+}
+
+// The 4 floats at byte offset off, of which the first n are in the operand.
+template <bool WIDE>
+__device__ __forceinline__ float4 f32_run(__amdgpu_buffer_rsrc_t rs, uint32_t off, int n) {
+  if (WIDE) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, n > 0 ? off : kOob, 0, 0);
+    return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z),
+                       __uint_as_float(v.w));
+  }
+  float v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    v[j] = __uint_as_float(
+        __builtin_amdgcn_raw_buffer_load_b32(rs, j < n ? off + 4 * j : kOob, 0, 0));
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+
+template <bool KCONTIG>
+struct VecOp {
+  const float* base;    // the tile's corner at k = 0
+  int64_t step;         // floats from one k to the next
+  uint32_t off[kRuns];  // bytes from base (+ k0 * step) of the thread's runs
+  int n[kRuns];         // KCONTIG: row inside; else elements of the run inside
+  __device__ __forceinline__ void init(const float* corner, int64_t ld, int64_t extent) {
+    base = corner;
+    step = KCONTIG ? 1 : ld;
+#pragma unroll
+    for (int i = 0; i < kRuns; ++i) {
+      int k, x;
+      run_at<KCONTIG>(i, k, x);
+      n[i] = (int)min<int64_t>(extent - x, 4);
+      off[i] = (uint32_t)((KCONTIG ? x * ld + k : k * ld + x) * 4);
+    }
+  }
+  template <bool WIDE>
+  __device__ __forceinline__ void load(float4 (&r)[kRuns], int64_t k0, int64_t K) const {
+    const auto rs = f32_rsrc(base + k0 * step);
+#pragma unroll
+    for (int i = 0; i < kRuns; ++i) {
+      int k, x;
+      run_at<KCONTIG>(i, k, x);
+      const int left = (int)min<int64_t>(K - k0 - k, 4);
+      r[i] = f32_run<WIDE>(rs, off[i], KCONTIG ? (n[i] > 0 ? left : 0) : (left > 0 ? n[i] : 0));
+    }
+  }
+};
+
+// Whether a launch's offsets from a tile's corner, or from the gathered matrix,
+// stay below 2^31 bytes and its gradient operand is stored as it is used (host).
+template <int F>
+bool f32_vec(const F32Args& p) {
+  if ((F == F_UP_DX || F == F_UP_DW) && p.act != VMOE_ACT_NONE) return false;
+  const int64_t la = F == F_UP_DX ? p.ldg : p.lda, lb = F == F_UP_DW ? p.ldg : p.ldb;
+  return la < (1 << 22) && lb < (1 << 22) && (!p.a_map || p.a_rows * la < (int64_t)1 << 29);
+}
+
+template <int F>
+__device__ __forceinline__ bool tile_wide(const F32Args& p, const F32Prob& q) {
+  const uint64_t bits =
+      reinterpret_cast<uint64_t>(a_src<F>(p)) | reinterpret_cast<uint64_t>(b_src<F>(p)) |
+      (uint64_t)((a_ld<F>(p) | b_ld<F>(p) | p.hidden | q.w | q.w0) * 4);
+  return (bits & 15) == 0;
 }
 
 // GLU: the SwiGLU up forward (a second accumulator over the up columns); its
-// own instance, so the other forms do not carry its registers.
-template <int F, bool GLU>
+// own instance, so the other forms do not carry its registers. VEC: f32_vec.
+template <int F, bool GLU, bool VEC>
 __global__ __launch_bounds__(kThreads) void grouped_gemm_f32_kernel(F32Args p) {
-  __shared__ __align__(16) float As[kBK][kPad];
-  __shared__ __align__(16) float Bs[kBK][kPad];
-  __shared__ __align__(16) float Us[GLU ? kBK : 1][kPad];  // SwiGLU up half
+  __shared__ __align__(16) float As[2][kStage];
+  __shared__ __align__(16) float Bs[2][kStage];
+  __shared__ __align__(16) float Us[2][GLU ? kStage : 4];  // SwiGLU up half
   constexpr bool glu = GLU && F == F_UP_FWD;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  int e = 0;
-  int64_t before = 0;  // tiles of experts < e
-  F32Prob q{};
-  int64_t tiles = 0, tn_count = 1;
-  bool have = false;
-  for (int64_t t = blockIdx.x;; t += gridDim.x) {
-    // experts are visited in order and t only grows, so one pass over them
-    while (true) {
-      if (!have) {
-        if (e >= p.E) break;
-        q = f32_prob<F>(p, e);
-        tn_count = cdiv64(q.N, kT);
-        tiles = cdiv64(q.M, kT) * tn_count;
-        have = true;
-      }
-      if (t < before + tiles) break;
-      before += tiles;
-      ++e;
-      have = false;
-    }
-    if (!have) break;
-    const int64_t local = t - before;
+  constexpr bool AK = a_k_contig<F>(), BKC = b_k_contig<F>();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  int e;
+  int64_t local;
+  for (int64_t j = blockIdx.x >> 3; find_tile<F>(p, j, e, local); j += gridDim.x >> 3) {
+    const F32Prob q = f32_prob<F>(p, e);
+    const int64_t tn_count = cdiv64(q.N, kT);
     const int64_t m0 = (local / tn_count) * kT, n0 = (local % tn_count) * kT;
-    float acc[4][4] = {}, acc_up[glu ? 4 : 1][4] = {};
-    for (int64_t k0 = 0; k0 < q.K; k0 += kBK) {
-      if constexpr (F == F_UP_DX)
-        stage_elem<true>(As, [&](int k, int x) { return f32_a<F>(p, q, m0 + x, k0 + k); });
-      else
-        stage<a_k_contig<F>()>(As, [&](int k, int x) { return f32_a_run<F>(p, q, m0 + x, k0 + k); });
-      if constexpr (F == F_UP_DW)
-        stage_elem<false>(Bs, [&](int k, int x) { return f32_b<F>(p, q, k0 + k, n0 + x, false); });
-      else
-        stage<b_k_contig<F>()>(Bs, [&](int k, int x) {
-          return f32_b_run<F>(p, q, k0 + k, n0 + x, false);
-        });
-      if constexpr (glu)
-        stage<false>(Us, [&](int k, int x) { return f32_b_run<F>(p, q, k0 + k, n0 + x, true); });
-      __syncthreads();
+    f32x16_t acc, acc_up;
 #pragma unroll
-      for (int k = 0; k < kBK; ++k) {
-        // each thread's 4 rows / 4 columns are consecutive: one 16-byte LDS
-        // read per operand (the 16 lanes of a row group read 256 contiguous
-        // bytes of B, and share one address of A)
-        const float4 av = *reinterpret_cast<const float4*>(&As[k][4 * ty]);
-        const float4 bv = *reinterpret_cast<const float4*>(&Bs[k][4 * tx]);
-        const float a[4] = {av.x, av.y, av.z, av.w};
-        float b[4] = {bv.x, bv.y, bv.z, bv.w};
+    for (int v = 0; v < 16; ++v) acc[v] = acc_up[v] = 0.0f;
+    float4 ra[kRuns], rb[kRuns], ru[glu ? kRuns : 1];
+    // Multiplies stage by stage, the next stage's loads in flight meanwhile;
+    // two LDS buffers, so one barrier per stage: a wave that has passed stage
+    // s's barrier has every wave behind it past stage s - 1's reads.
+    auto multiply = [&](auto&& load) {
+      int buf = 0;
+      if (q.K > 0) load(0);
+      for (int64_t k0 = 0; k0 < q.K; k0 += kBK, buf ^= 1) {
+        store_stage<AK>(As[buf], ra);
+        store_stage<BKC>(Bs[buf], rb);
+        if constexpr (glu) store_stage<BKC>(Us[buf], ru);
+        __syncthreads();
+        if (k0 + kBK < q.K) load(k0 + kBK);
+        float4 fa[kBK / 8], fb[kBK / 8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int u = 0; u < kBK / 8; ++u) {
+          fa[u] = frag<AK>(As[buf], wm, 8 * u);
+          fb[u] = frag<BKC>(Bs[buf], wn, 8 * u);
+        }
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-        if constexpr (glu) {
-          const float4 uv = *reinterpret_cast<const float4*>(&Us[k][4 * tx]);
-          b[0] = uv.x; b[1] = uv.y; b[2] = uv.z; b[3] = uv.w;
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc_up[i][j] = fmaf(a[i], b[j], acc_up[i][j]);
+        for (int u = 0; u < kBK / 8; ++u) {
+          mfma4(acc, fa[u], fb[u]);
+          if constexpr (glu) mfma4(acc_up, fa[u], frag<BKC>(Us[buf], wn, 8 * u));
         }
       }
-      __syncthreads();
-    }
+      __syncthreads();  // before the next tile's first stage
+    };
+    if constexpr (VEC) {
+      const bool wide = tile_wide<F>(p, q);
+      VecOp<AK> va;
+      VecOp<BKC> vb, vu;
+      const float* a = a_src<F>(p);
+      const float* b = b_src<F>(p);
+      const int64_t la = a_ld<F>(p), lb = b_ld<F>(p);
+      const int32_t* map = F == F_UP_FWD || F == F_UP_DW ? p.a_map : nullptr;
+      va.init(map ? a + (AK ? 0 : m0) : a + (AK ? (q.t0 + m0) * la : q.t0 * la + m0), la,
+              q.M - m0);
+      if constexpr (F == F_UP_FWD) {
+        if (map) {  // the rows of the tile, the same for every stage
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t m = m0 + 4 * ty + i;
-      if (m >= q.M) continue;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t n = n0 + 4 * tx + j;
-        if (n >= q.N) continue;
-        const float z = acc[i][j];
-        if (F == F_UP_DW) {
-          p.c[m * p.ldc + q.w0 + n] = z;
-        } else if (F == F_DOWN_DW) {
-          p.c[(q.w0 + m) * p.ldc + n] = z;
-        } else {
-          const int64_t o = (q.t0 + m) * p.ldc + n;
-          if (F == F_UP_FWD && p.act == VMOE_ACT_RELU_SQUARED) {
-            const float r = fmaxf(z, 0.0f);
-            if (p.c2) p.c2[o] = r;
-            p.c[o] = r * r;
-          } else if constexpr (glu) {
-            const float u = acc_up[i][j];
-            if (p.c2) p.c2[o] = z;
-            if (p.c3) p.c3[o] = u;
-            if (p.c) p.c[o] = z * sigmoid32(z) * u;
-          } else {
-            p.c[o] = z;
+          for (int i = 0; i < kRuns; ++i) {
+            int k, x;
+            run_at<true>(i, k, x);
+            const int64_t s = m0 + x < q.M ? map[q.t0 + m0 + x] : -1;
+            va.n[i] = s >= 0 && s < p.a_rows ? 4 : 0;
+            va.off[i] = (uint32_t)((s * la + k) * 4);
           }
+        }
+      }
+      switch (F) {
+        case F_UP_FWD: vb.init(b + q.w0 + n0, lb, q.N - n0); break;
+        case F_DOWN_FWD: vb.init(b + q.w0 * lb + n0, lb, q.N - n0); break;
+        case F_UP_DX: vb.init(b + n0 * lb + q.w0, lb, q.N - n0); break;
+        case F_DOWN_DH: vb.init(b + (q.w0 + n0) * lb, lb, q.N - n0); break;
+        default: vb.init(b + q.t0 * lb + n0, lb, q.N - n0); break;  // both dW
+      }
+      if constexpr (glu) vu.init(b + q.w0 + q.w + n0, lb, q.N - n0);
+      if (F == F_UP_DW && map) {
+        // gathered token rows as K: each stage's map entries are read a stage
+        // ahead of its rows
+        int32_t tok[kRuns];
+        auto entries = [&](int64_t k0) {
+#pragma unroll
+          for (int i = 0; i < kRuns; ++i) {
+            int k, x;
+            run_at<false>(i, k, x);
+            tok[i] = k0 + k < q.K ? map[q.t0 + k0 + k] : -1;
+          }
+        };
+        entries(0);
+        const auto rs = f32_rsrc(va.base);
+        auto run = [&](auto w) {
+          constexpr bool WIDE = decltype(w)::value;
+          multiply([&](int64_t k0) {
+#pragma unroll
+            for (int i = 0; i < kRuns; ++i) {
+              int k, x;
+              run_at<false>(i, k, x);
+              const bool ok = tok[i] >= 0 && tok[i] < p.a_rows;
+              ra[i] = f32_run<WIDE>(rs, (uint32_t)((tok[i] * la + x) * 4), ok ? va.n[i] : 0);
+            }
+            entries(k0 + kBK);
+            vb.template load<WIDE>(rb, k0, q.K);
+          });
+        };
+        if (wide) run(std::true_type{}); else run(std::false_type{});
+      } else {
+        auto run = [&](auto w) {
+          constexpr bool WIDE = decltype(w)::value;
+          multiply([&](int64_t k0) {
+            va.template load<WIDE>(ra, k0, q.K);
+            vb.template load<WIDE>(rb, k0, q.K);
+            if constexpr (glu) vu.template load<WIDE>(ru, k0, q.K);
+          });
+        };
+        if (wide) run(std::true_type{}); else run(std::false_type{});
+      }
+    } else {
+      multiply([&](int64_t k0) {
+        if (F == F_UP_DX && p.act != VMOE_ACT_NONE)
+          load_stage<AK>(ra, [&](int k, int x) {
+            return make_float4(f32_a<F>(p, q, m0 + x, k0 + k), f32_a<F>(p, q, m0 + x, k0 + k + 1),
+                               f32_a<F>(p, q, m0 + x, k0 + k + 2),
+                               f32_a<F>(p, q, m0 + x, k0 + k + 3));
+          });
+        else
+          load_stage<AK>(ra, [&](int k, int x) { return f32_a_run<F>(p, q, m0 + x, k0 + k); });
+        if (F == F_UP_DW && p.act != VMOE_ACT_NONE)
+          load_stage<BKC>(rb, [&](int k, int x) {
+            return make_float4(f32_b<F>(p, q, k0 + k, n0 + x, false),
+                               f32_b<F>(p, q, k0 + k, n0 + x + 1, false),
+                               f32_b<F>(p, q, k0 + k, n0 + x + 2, false),
+                               f32_b<F>(p, q, k0 + k, n0 + x + 3, false));
+          });
+        else
+          load_stage<BKC>(rb,
+                          [&](int k, int x) { return f32_b_run<F>(p, q, k0 + k, n0 + x, false); });
+        if constexpr (glu)
+          load_stage<BKC>(ru,
+                          [&](int k, int x) { return f32_b_run<F>(p, q, k0 + k, n0 + x, true); });
+      });
+    }
+    // acc[v]: row 8 (v / 4) + 4 (lane / 32) + v % 4, column lane % 32 of the block
+    const int64_t n = n0 + wn + (lane & 31);
+    if (n >= q.N) continue;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int64_t m = m0 + wm + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+      if (m >= q.M) continue;
+      const float z = acc[v];
+      if (F == F_UP_DW) {
+        p.c[m * p.ldc + q.w0 + n] = z;
+      } else if (F == F_DOWN_DW) {
+        p.c[(q.w0 + m) * p.ldc + n] = z;
+      } else {
+        const int64_t o = (q.t0 + m) * p.ldc + n;
+        if (F == F_UP_FWD && p.act == VMOE_ACT_RELU_SQUARED) {
+          const float r = fmaxf(z, 0.0f);
+          if (p.c2) p.c2[o] = r;
+          p.c[o] = r * r;
+        } else if constexpr (glu) {
+          const float u = acc_up[v];
+          if (p.c2) p.c2[o] = z;
+          if (p.c3) p.c3[o] = u;
+          if (p.c) p.c[o] = z * sigmoid32(z) * u;
+        } else {
+          p.c[o] = z;
         }
       }
     }
@@ -370,9 +597,16 @@ int64_t tile_bound(int64_t E, int64_t m_bound, int64_t n_bound, bool rows_m) {
 template <int F, bool GLU = false>
 int f32_launch(const F32Args& p, int64_t bound, hipStream_t s) {
   if (bound <= 0 || p.rows_bound == 0 || p.max_width == 0) return VMOE_OK;  // no work
-  const int64_t grid = bound < 2048 ? bound : 2048;
-  VMOE_LAUNCH((grouped_gemm_f32_kernel<F, GLU>), dim3((unsigned)grid), dim3(kThreads), 0, s,
-                     p);
+  // one workgroup per tile in eight XCD ranges (find_tile), so that the
+  // hardware deals tiles of unequal K to free slots; past the real count they
+  // leave at once
+  const int64_t grid = std::min<int64_t>((bound + 7) / 8 * 8, 1 << 22);
+  if (f32_vec<F>(p))
+    VMOE_LAUNCH((grouped_gemm_f32_kernel<F, GLU, true>), dim3((unsigned)grid), dim3(kThreads), 0,
+                s, p);
+  else
+    VMOE_LAUNCH((grouped_gemm_f32_kernel<F, GLU, false>), dim3((unsigned)grid), dim3(kThreads), 0,
+                s, p);
   VMOE_CHECK_LAUNCH();
   return VMOE_OK;
 }

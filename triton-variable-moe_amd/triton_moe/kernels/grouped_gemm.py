@@ -445,7 +445,7 @@ def down_bwd(grad_y, h, w2, m: GemmMeta, hidden: int, zero_tails: bool,
 # ---------------------------------------------------------------------------
 # fp32 path: float32 weights (the reference's kernels are dtype-generic and
 # its autograd tests run fp32, tests/test_grouped_gemm_backward.py:151-208).
-# One fp32 VALU kernel per GEMM form (csrc/gemm_f32.hip); outputs are fp32
+# One fp32 MFMA kernel per GEMM form (csrc/gemm_f32.hip); outputs are fp32
 # and zero outside the rows and columns the experts cover.
 # ---------------------------------------------------------------------------
 
@@ -465,8 +465,24 @@ def _f32(t: torch.Tensor, what: str) -> torch.Tensor:
     return t if ok else t.contiguous()
 
 
-def _f32_zeros(rows, cols, device):
-    return torch.zeros(rows, cols, dtype=torch.float32, device=device)
+def _f32_out(rows, cols, device, zero):
+    """An output of the fp32 kernels, zero-filled where they leave part of it
+    unwritten: rows no tile covers, columns past an expert's width, a launch
+    without work."""
+    f = torch.zeros if zero else torch.empty
+    return f(rows, cols, dtype=torch.float32, device=device)
+
+
+def _f32_rows_left(m: GemmMeta) -> bool:
+    return not m.full_rows or m.max_width == 0
+
+
+def _f32_inter_left(m: GemmMeta) -> bool:
+    return not m.full_rows or not m.uniform
+
+
+def _f32_weights_left(m: GemmMeta) -> bool:
+    return not m.full_cols or m.rows == 0 or m.max_width == 0
 
 
 def f32_up_fwd(x, w1, m: GemmMeta, act: int, gather_map=None, want_out=True, want_pre=False,
@@ -482,9 +498,12 @@ def f32_up_fwd(x, w1, m: GemmMeta, act: int, gather_map=None, want_out=True, wan
     else:
         _need(gather_map.numel() >= m.rows, "gather_map shorter than the padded row count")
     dev = x.device
-    out = _f32_zeros(m.rows, m.max_width, dev) if want_out else None
-    pre = _f32_zeros(m.rows, m.max_width, dev) if want_pre else None
-    up = _f32_zeros(m.rows, m.max_width, dev) if want_up and act == ACT_SWIGLU else None
+    left = _f32_inter_left(m)
+    out = _f32_out(m.rows, m.max_width, dev, left) if want_out else None
+    # without an activation the kernel writes no pre: zeros, as ever
+    pre = (_f32_out(m.rows, m.max_width, dev, left or act == _lib.ACT_NONE) if want_pre
+           else None)
+    up = _f32_out(m.rows, m.max_width, dev, left) if want_up and act == ACT_SWIGLU else None
     gm = None if gather_map is None else _i32(gather_map)
     if m.rows > 0:
         _lib.call("vmoe_gemm_f32_up_fwd", x.data_ptr(), x.stride(0), x.shape[0], _lib.ptr(gm),
@@ -500,7 +519,7 @@ def f32_down_fwd(h, w2, m: GemmMeta, hidden: int):
     _need(w2.shape[1] == hidden, "w2 columns must equal hidden_size")
     _need(h.shape[0] >= m.rows and h.shape[1] >= m.max_width,
           "intermediate smaller than [rows, max_expert_width]")
-    y = _f32_zeros(m.rows, hidden, h.device)
+    y = _f32_out(m.rows, hidden, h.device, _f32_rows_left(m))
     if m.rows > 0:
         _lib.call("vmoe_gemm_f32_down_fwd", h.data_ptr(), h.stride(0), w2.data_ptr(),
                   w2.stride(0), y.data_ptr(), y.stride(0), *_meta_args(m), hidden, m.max_width,
@@ -532,8 +551,8 @@ def f32_up_bwd(grad_h, x, w1, pre, up, m: GemmMeta, hidden: int, act: int, gathe
     else:
         _need(gather_map.numel() >= m.rows, "gather_map shorter than the padded row count")
     dev = grad_h.device
-    grad_x = _f32_zeros(m.rows, hidden, dev)
-    grad_w1 = torch.zeros(w1.shape, dtype=torch.float32, device=dev)
+    grad_x = _f32_out(m.rows, hidden, dev, _f32_rows_left(m))
+    grad_w1 = _f32_out(*w1.shape, dev, _f32_weights_left(m))
     gm = None if gather_map is None else _i32(gather_map)
     g, p_, u = ops
     if act == _lib.ACT_RELU_SQUARED and g.numel() > 0:
@@ -565,8 +584,8 @@ def f32_down_bwd(grad_y, h, w2, m: GemmMeta, hidden: int):
     _need(h.shape[0] >= m.rows and h.shape[1] >= m.max_width,
           "intermediate smaller than [rows, max_expert_width]")
     dev = grad_y.device
-    grad_h = _f32_zeros(m.rows, m.max_width, dev)
-    grad_w2 = torch.zeros(w2.shape, dtype=torch.float32, device=dev)
+    grad_h = _f32_out(m.rows, m.max_width, dev, _f32_inter_left(m))
+    grad_w2 = _f32_out(*w2.shape, dev, _f32_weights_left(m))
     if m.rows > 0:
         _lib.call("vmoe_gemm_f32_down_bwd_dh", grad_y.data_ptr(), grad_y.stride(0),
                   w2.data_ptr(), w2.stride(0), grad_h.data_ptr(), grad_h.stride(0),

@@ -39,8 +39,11 @@ CASES = [
     # hidden and widths multiples of 8 only: every K loop ends in a partial
     # stage (K = 200 or a width of 40 / 24 / 8), top_k 1
     (300, 200, [(3, 40), (2, 24), (1, 8)], 1, 64, False),
+    # 284 up tiles: one round of 256 CUs and a last one whose tiles are cut
+    (300, 256, [(66, 1024), (6, 576), (2, 64)], 2, 64, False),
 ]
-IDS = ["small", "uniform", "variable", "tiny_tiles", "var3", "skew64", "wide_lanes8", "mult8"]
+IDS = ["small", "uniform", "variable", "tiny_tiles", "var3", "skew64", "wide_lanes8", "mult8",
+       "cut_round"]
 
 
 def _case(T, d, sizes, k, b, skew, seed=0):
@@ -747,3 +750,29 @@ def test_column_slice_operands(device):
     torch.cuda.synchronize()
     for a, b in zip(*res):
         assert bits_equal(a, b)
+
+
+@pytest.mark.parametrize("activation,widths", [("relu_squared", [1000] * 70),
+                                               ("swiglu", [488] * 70)])
+def test_cut_last_round_same_bits(activation, widths, device):
+    """280 tiles (one round of 256 CUs and 24 tiles cut into column pieces; the
+    widths end inside a piece) give the bits of the same experts in two calls
+    of 140 tiles, which cut none."""
+    E, d, w, rows = len(widths), 136, widths[0], 8
+    mult = 2 if activation == "swiglu" else 1
+    g = torch.Generator().manual_seed(11)
+    x = torch.randn(E * rows, d, generator=g).to(torch.bfloat16).to(device)
+    w1 = (torch.randn(d, E * w * mult, generator=g) * 0.05).to(torch.bfloat16).to(device)
+
+    def up(e0, e1):
+        n = e1 - e0
+        i32 = dict(dtype=torch.int32, device=device)
+        eto = torch.arange(0, n * rows + 1, rows, **i32)
+        ewo = torch.arange(e0 * w * mult, e1 * w * mult + 1, w * mult, **i32)
+        return grouped_gemm_up(x[e0 * rows:e1 * rows], w1, eto, ewo, torch.full((n,), w, **i32),
+                               torch.full((n,), rows, **i32), w, activation=activation,
+                               save_pre_act=True)
+
+    whole, parts = up(0, E), [up(0, E // 2), up(E // 2, E)]
+    for i in range(2):
+        assert bits_equal(whole[i], torch.cat([p[i] for p in parts]))

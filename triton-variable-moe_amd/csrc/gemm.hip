@@ -433,6 +433,25 @@ struct Meta {
 // partial slots.
 struct Range {
   int beg, end, stride, lin, slot;
+  // Round-robin: where an XCD's tiles are one round and up to a quarter of
+  // another, the tiles of that second round are cut along n into cut = 4
+  // pieces, so that four times as many workgroups share it; this workgroup
+  // takes piece `piece` of tile `tail` (-1: none). cut is 1 otherwise. A piece
+  // takes as many k-steps and staging instructions as its tile and a quarter
+  // of the bytes of B, so it pays where the GEMM streams weights (few rows per
+  // expert: 1531 tokens through 128 experts of 256-1024, up projection 104 ->
+  // 89 us); a step bound by staging (8192 tokens through 8 experts of 512)
+  // takes the same time with and without. After more rounds, or for a fuller
+  // last one (halves), it cost up to 1 %; with no full round before it (64
+  // tokens, 64 experts of 256) 20.3 -> 22.0 us.
+  int tail, piece, cut;
+  // The workgroup's items in order: beg, beg + stride, ... below end, then the
+  // tail; -1 past the last.
+  __device__ __forceinline__ int first() const { return beg < end ? beg : tail; }
+  __device__ __forceinline__ int next(int item) const {
+    return item >= end ? -1 : item + stride < end ? item + stride : tail;
+  }
+  __device__ __forceinline__ int cut_of(int item) const { return item < end ? 1 : cut; }
 };
 
 // The workgroup's index among the p.grid workgroups of its GEMM. A paired
@@ -460,10 +479,19 @@ __device__ __forceinline__ Range item_range(const Args& p, int total, const int*
     r.beg = lane_beg[lane];
     r.end = lane_beg[lane + 1];
     r.stride = 1;
+    r.tail = -1;
+    r.piece = 0;
+    r.cut = 1;
   } else {
-    r.beg = lane_beg[xcd] + j;
-    r.end = lane_beg[xcd + 1];
+    const int first = __builtin_amdgcn_readfirstlane(lane_beg[xcd]);
+    const int count = __builtin_amdgcn_readfirstlane(lane_beg[xcd + 1]) - first;
+    const int rounds = udiv_small(count, per), rem = count - rounds * per;
+    r.cut = rounds == 1 && 4 * rem <= per ? 4 : 1;
+    r.beg = first + j;
+    r.end = r.cut > 1 ? first + rounds * per : first + count;
     r.stride = per;
+    r.tail = r.cut > 1 && j < 4 * rem ? r.end + (j >> 2) : -1;
+    r.piece = j & 3;
   }
   return r;
 }
@@ -916,6 +944,7 @@ struct Gemm {
 
   struct Work {
     int m0, n0, kbeg, klen, nk, chunk, chunks;
+    int nend;   // columns of the problem at or past this are not this item's
     bool skip;  // contig: the item's tile group has no tile for this slot
     Prob q;
   };
@@ -924,7 +953,9 @@ struct Gemm {
   // expert with a wave-wide search of the prefix table from the cursor, then
   // its tile (for contig, that of lane slot `slot`) and K chunk. Every field
   // is workgroup-uniform.
-  __device__ static Work decode(const Args& p, const Meta& mt, int item, int& ecur, int slot) {
+  // piece of cut: the item's share of the tile's columns (see Range).
+  __device__ static Work decode(const Args& p, const Meta& mt, int item, int& ecur, int slot,
+                                int piece = 0, int cut = 1) {
     const int lane = threadIdx.x & 63;
     int e = ecur;
     for (;;) {
@@ -964,6 +995,13 @@ struct Gemm {
     const int mt_idx = n_tiles == 1 ? tile : udiv_small(tile, n_tiles);
     w.m0 = mt_idx * BM;
     w.n0 = (tile - mt_idx * n_tiles) * BNO;
+    w.nend = w.q.N;
+    if (!Cfg<V>::contig && cut > 1) {
+      const int cols = BNO / 4;
+      w.n0 += piece * cols;
+      w.nend = min(w.q.N, w.n0 + cols);
+      w.skip |= w.n0 >= w.q.N;
+    }
     w.kbeg = 0;
     w.chunk = chunk;
     w.chunks = chunks;
@@ -1002,13 +1040,13 @@ struct Gemm {
       setup_t<BM, PWA, T::t_map>(sa, tm, p.a, p.lda, p.a_map, p.a_rows, q.ar + w.kbeg,
                                  q.ac + w.m0, q.M - w.m0, w.klen, !T::t_map_b);
     if (V == UP_GLU)
-      setup_glu(sb, p.b, p.ldb, q.br + w.kbeg, q.bc + w.n0, q.N, q.N - w.n0);
+      setup_glu(sb, p.b, p.ldb, q.br + w.kbeg, q.bc + w.n0, q.N, w.nend - w.n0);
     else if (T::b_k)
-      setup_k<BN, PWB, false>(sb, p.b, p.ldb, nullptr, 0, q.br + w.n0, q.bc + w.kbeg, q.N - w.n0,
-                              nullptr);
+      setup_k<BN, PWB, false>(sb, p.b, p.ldb, nullptr, 0, q.br + w.n0, q.bc + w.kbeg,
+                              w.nend - w.n0, nullptr);
     else
       setup_t<BN, PWB, T::t_map_b>(sb, tm, p.b, p.ldb, p.b_map, p.b_rows, q.br + w.kbeg,
-                                   q.bc + w.n0, q.N - w.n0, w.klen, T::t_map_b);
+                                   q.bc + w.n0, w.nend - w.n0, w.klen, T::t_map_b);
   }
 
   // Issues k-step kt of item w as global stage s (A of a pair: on even kt).
@@ -1181,7 +1219,7 @@ struct Gemm {
     }
     pd.mb = w.m0 + wm * WM;
     pd.nb = w.n0 + wn * (V == UP_GLU ? WN / 2 : WN);
-    pd.M = q.M; pd.N = q.N; pd.cr = q.cr; pd.cc = q.cc;
+    pd.M = q.M; pd.N = w.nend; pd.cr = q.cr; pd.cc = q.cc;
     if constexpr (V == UP_GLU) {
       // Block j = 0 holds the gate g, j = 1 the up projection u of the same
       // 32 outputs: gate and up (bf16) go to unit (0, i), H = bf16(g
@@ -1513,7 +1551,7 @@ struct Gemm {
     int win_stage = -2;     // the same for the current item's window
     int done = -2;          // every DMA issued before stage done + 1's is complete
     int issued = 0;         // stages issued
-    int ikt = 0, inext = rg.beg, witem = rg.beg;
+    int ikt = 0, inext = rg.first(), witem = -1;
     Work wla;  // decode of la_item, reused when that item begins
     auto begin_item = [&]() {
       if (mapped) {
@@ -1550,8 +1588,8 @@ struct Gemm {
       ++nbegun;
       if (!mapped) return;
       la_item = -1;
-      for (int nx = witem + rg.stride; nx < rg.end; nx += rg.stride) {
-        wla = decode(p, mt, nx, ela, rg.slot);
+      for (int nx = rg.next(witem); nx >= 0; nx = rg.next(nx)) {
+        wla = decode(p, mt, nx, ela, rg.slot, rg.piece, rg.cut_of(nx));
         if (wla.nk > 0) {
           TMap tn = tm;
           setup_map(p, wla, tn);
@@ -1565,10 +1603,11 @@ struct Gemm {
     // Moves to the next item with k-steps and sets it up (decode, operand
     // offsets, row factors, the next map window); false at the range's end.
     auto advance = [&]() -> bool {
-      while (inext < rg.end) {
+      while (inext >= 0) {
         witem = inext;
-        wi = inext == la_item ? wla : decode(p, mt, inext, ei, rg.slot);
-        inext += rg.stride;
+        wi = inext == la_item ? wla
+                              : decode(p, mt, inext, ei, rg.slot, rg.piece, rg.cut_of(inext));
+        inext = rg.next(inext);
         if (wi.nk > 0) {
           ikt = 0;
           begin_item();
@@ -1638,8 +1677,8 @@ struct Gemm {
     for (int qq = 0; qq < 4; ++qq) pr[qq] = make_uint4(0, 0, 0, 0);
     // Units flush kLead k-steps after their PRE loads are issued.
     constexpr int kLead = V == DOWN_DH ? 2 : 0;
-    for (int item = rg.beg; item < rg.end; item += rg.stride) {
-      const Work w = decode(p, mt, item, ec, rg.slot);
+    for (int item = rg.first(); item >= 0; item = rg.next(item)) {
+      const Work w = decode(p, mt, item, ec, rg.slot, rg.piece, rg.cut_of(item));
       if (w.skip) continue;
       int slot = 0;
       if constexpr (kScaled) {
@@ -1725,7 +1764,7 @@ struct Gemm {
     const int total = build_meta(p, mt, (long long*)(char*)ring,
                                  (__attribute__((address_space(3))) int*)(ring + 256));
     const Range rg = item_range<Cfg<V>::contig>(p, total, mt.lane_beg);
-    if (rg.beg >= rg.end) return;
+    if (rg.first() < 0) return;
     const int wave = threadIdx.x >> 6;
     if (wave >= kConsumers)
       run_producer(p, ring, wins, scl, mt, rg);

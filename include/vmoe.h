@@ -749,6 +749,33 @@ int vmoe_moe_backward(const void* saved, const uint16_t* logits, int64_t num_tok
                       void* scratch, void* dw_workspace, size_t dw_workspace_bytes,
                       vmoe_stream_t stream, vmoe_stream_t side_stream);
 
+/* The float32 layer after its router Linear, one call per direction, as
+ * vmoe_moe_forward / vmoe_moe_backward are for bf16: fp32 logits [T, E]
+ * (contiguous; 16-byte aligned where E % 8 == 0), x, weights, losses and
+ * gradients; the routing weights go on the down projection's rows in the
+ * combine (scatter.py:106-133) and get no gradient. vmoe_moe_f32_layout:
+ * out[0..2] = bytes of saved, forward scratch and backward scratch.
+ * grad_out / grad_logits nullable as above; ldg may be 0 (one row for all). */
+int vmoe_moe_f32_layout(int64_t num_tokens, int32_t num_experts, int32_t top_k,
+                        int32_t block_size, int64_t hidden, int64_t max_width,
+                        int64_t* out /* [3] */);
+int vmoe_moe_f32_forward(const float* logits, int64_t num_tokens, int32_t num_experts,
+                         int32_t top_k, int32_t normalize, int32_t block_size, const float* x,
+                         int64_t ldx, const float* w1, int64_t ldw1, const float* w2,
+                         int64_t ldw2, const int32_t* ewo, const int32_t* widths, int64_t hidden,
+                         int64_t max_width, const float* coef, const float* widths_normalized,
+                         void* saved, void* scratch, float* out, int64_t ldo, float* z_loss,
+                         float* losses, float* f_i, vmoe_stream_t stream);
+int vmoe_moe_f32_backward(const void* saved, const float* logits, int64_t num_tokens,
+                          int32_t num_experts, int32_t top_k, int32_t block_size, const float* x,
+                          int64_t ldx, const float* w1, int64_t ldw1, const float* w2,
+                          int64_t ldw2, const int32_t* ewo, const int32_t* widths, int64_t hidden,
+                          int64_t max_width, const float* coef, const float* widths_normalized,
+                          const float* grad_out, int64_t ldg, const float* grad_z,
+                          const float* grad_lb, const float* grad_cl, float* grad_x, int64_t ldgx,
+                          float* grad_w1, int64_t ldgw1, float* grad_w2, int64_t ldgw2,
+                          float* grad_logits, void* scratch, vmoe_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

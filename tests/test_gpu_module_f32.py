@@ -197,3 +197,36 @@ def test_f32_training_tracks_oracle(device):
                                                                           loss_t.item())
     assert_close_norm(m.w1.detach(), twin_w1.detach(), F32_TOL, "w1 after 10 steps")
     assert_close_norm(m.w2.detach(), twin_w2.detach(), F32_TOL, "w2 after 10 steps")
+
+
+@pytest.mark.parametrize("name", ["validate_training", "ref_variable", "k8_64", "unaligned"])
+@pytest.mark.parametrize("grad", ["dense", "sum", "aux_only"])
+def test_f32_one_call_path_same_bits_as_per_kernel_path(name, grad, device):
+    """The one-node float32 layer (one library call per direction) gives the
+    bits of the per-kernel path: outputs, losses, f_i and every gradient, for
+    a dense gradient, out.sum()'s broadcast one, and the losses alone."""
+    from triton_moe.kernels import grouped_gemm as gg
+
+    B, S, d, sizes, k, b = SHAPES[name]
+    g = torch.Generator().manual_seed(3)
+    x0 = torch.randn(B, S, d, generator=g).to(device)
+    G = torch.randn(B, S, d, generator=g).to(device)
+    got = []
+    for fused in (True, False):
+        gg.FUSED_EXPERT_PATH = fused
+        try:
+            m = _model(d, sizes, k, b, device)
+            x = x0.clone().requires_grad_(True)
+            out, aux, f_i = m(x)
+            losses = aux["router_z_loss"] + aux["load_balance_loss"] + aux["compute_loss"]
+            if grad == "aux_only":
+                losses.backward()
+            else:
+                ((out * G).sum() + losses if grad == "dense" else out.sum()).backward()
+            got.append([out, f_i, *aux.values(), x.grad, m.router.weight.grad, m.w1.grad,
+                        m.w2.grad])
+        finally:
+            gg.FUSED_EXPERT_PATH = True
+    for a, c in zip(*got):
+        assert (a is None) == (c is None)
+        assert a is None or (a.dtype == c.dtype and torch.equal(a, c))

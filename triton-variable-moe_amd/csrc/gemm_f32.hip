@@ -578,6 +578,9 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_f32_kernel(F32Args p) {
           if (p.c2) p.c2[o] = z;
           if (p.c3) p.c3[o] = u;
           if (p.c) p.c[o] = z * sigmoid32(z) * u;
+        } else if (F == F_DOWN_DH && p.pre) {
+          const float pr = p.pre[o];  // the relu^2 rule (pre shares c's layout)
+          p.c[o] = pr > 0.0f ? z * 2.0f * pr : 0.0f;
         } else {
           p.c[o] = z;
         }
@@ -760,23 +763,34 @@ extern "C" int vmoe_gemm_f32_up_bwd_dw(const float* x, int64_t ldx, int64_t x_ro
                              reinterpret_cast<hipStream_t>(stream));
 }
 
+namespace vmoe {
+int gemm_f32_down_bwd_ga(const float* grad_y, int64_t ldgy, const float* w2, int64_t ldw2,
+                         const float* pre_act, float* ga, int64_t ldga, const int32_t* eto,
+                         const int32_t* ewo, const int32_t* widths, const int32_t* tpe, int32_t E,
+                         int64_t hidden, int64_t max_width, int64_t rows_bound,
+                         vmoe_stream_t stream) {
+  int st = f32_common(eto, ewo, widths, tpe, E, hidden, max_width, rows_bound);
+  if (st) return st;
+  if (!grad_y || ldgy < hidden || !w2 || ldw2 < hidden || !ga || ldga < max_width || ldga <= 0)
+    return VMOE_ERR_INVALID_ARG;
+  F32Args p = f32_args(eto, ewo, widths, tpe, E, hidden, max_width, rows_bound, VMOE_ACT_NONE);
+  p.a = grad_y; p.lda = ldgy;
+  p.b = w2; p.ldb = ldw2;
+  p.pre = pre_act;
+  p.c = ga; p.ldc = ldga;
+  return f32_launch<F_DOWN_DH>(p, tile_bound(E, rows_bound, max_width, true),
+                               reinterpret_cast<hipStream_t>(stream));
+}
+}  // namespace vmoe
+
 extern "C" int vmoe_gemm_f32_down_bwd_dh(const float* grad_y, int64_t ldgy, const float* w2,
                                          int64_t ldw2, float* grad_h, int64_t ldgh,
                                          const int32_t* eto, const int32_t* ewo,
                                          const int32_t* widths, const int32_t* tpe, int32_t E,
                                          int64_t hidden, int64_t max_width, int64_t rows_bound,
                                          vmoe_stream_t stream) {
-  int st = f32_common(eto, ewo, widths, tpe, E, hidden, max_width, rows_bound);
-  if (st) return st;
-  if (!grad_y || ldgy < hidden || !w2 || ldw2 < hidden || !grad_h || ldgh < max_width ||
-      ldgh <= 0)
-    return VMOE_ERR_INVALID_ARG;
-  F32Args p = f32_args(eto, ewo, widths, tpe, E, hidden, max_width, rows_bound, VMOE_ACT_NONE);
-  p.a = grad_y; p.lda = ldgy;
-  p.b = w2; p.ldb = ldw2;
-  p.c = grad_h; p.ldc = ldgh;
-  return f32_launch<F_DOWN_DH>(p, tile_bound(E, rows_bound, max_width, true),
-                               reinterpret_cast<hipStream_t>(stream));
+  return gemm_f32_down_bwd_ga(grad_y, ldgy, w2, ldw2, nullptr, grad_h, ldgh, eto, ewo, widths, tpe,
+                              E, hidden, max_width, rows_bound, stream);
 }
 
 extern "C" int vmoe_gemm_f32_down_bwd_dw(const float* h, int64_t ldh, const float* grad_y,

@@ -35,6 +35,15 @@ extern thread_local LaunchTiming g_launch_timing;
 void gemm_pair_begin();
 int gemm_pair_end();
 
+// gemm_f32.hip: vmoe_gemm_f32_down_bwd_dh with the relu^2 rule in the epilogue,
+// ga = pre > 0 ? 2 gh pre : 0 for gh = grad_y W2_e^T (pre and ga share ldga):
+// the values vmoe_f32_relu2_grad forms from a stored gh.
+int gemm_f32_down_bwd_ga(const float* grad_y, int64_t ldgy, const float* w2, int64_t ldw2,
+                         const float* pre_act, float* ga, int64_t ldga, const int32_t* eto,
+                         const int32_t* ewo, const int32_t* widths, const int32_t* tpe, int32_t E,
+                         int64_t hidden, int64_t max_width, int64_t rows_bound,
+                         vmoe_stream_t stream);
+
 }  // namespace vmoe
 
 #define VMOE_LAUNCH(K, G, B, SH, S, ...)                                                   \

@@ -29,7 +29,7 @@ from torch.amp import custom_bwd, custom_fwd
 from torch.autograd.function import once_differentiable
 
 from .. import _lib
-from .gather import row_maps
+from .gather import _broadcast_rows, row_maps
 from .router import router_bwd
 
 _ACTIVATIONS = {"none": _lib.ACT_NONE, "relu_squared": _lib.ACT_RELU_SQUARED}
@@ -1246,10 +1246,7 @@ def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts):
     dev = logits.device
     plan = _moe_plan(T, E, k, b, d, max_width, dev)
 
-    def scalar(g):
-        return None if g is None else g.detach().to(torch.float32).reshape(()).contiguous()
-
-    gz, glb, gcl = scalar(g_z), scalar(g_lb), scalar(g_cl)
+    gz, glb, gcl = _scalar_f32(g_z), _scalar_f32(g_lb), _scalar_f32(g_cl)
     want_x = grad_out is not None and need_experts
     want_logits = need_logits and (
         gz is not None or glb is not None or gcl is not None or (weight_grad and want_x))
@@ -1289,6 +1286,102 @@ def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts):
     if st != _lib.OK:
         _lib.check(st, "vmoe_moe_backward")
     return grad_logits, grad_x, grad_w1, grad_w2
+
+
+def _scalar_f32(g):
+    """A loss gradient as the device fp32 scalar the kernels read (None: none)."""
+    return None if g is None else g.detach().to(torch.float32).reshape(()).contiguous()
+
+
+_MOE_F32_PLANS: dict[tuple, tuple] = {}
+
+
+def _moe_f32_plan(T, E, k, block_size, hidden, max_width) -> tuple:
+    """(saved, forward scratch, backward scratch) bytes and the two functions."""
+    key = (T, E, k, block_size, hidden, max_width)
+    plan = _MOE_F32_PLANS.get(key)
+    if plan is None:
+        out = (ctypes.c_int64 * 3)()
+        L = _lib.lib()
+        _lib.check(L.vmoe_moe_f32_layout(T, E, k, block_size, hidden, max_width, out),
+                   "vmoe_moe_f32_layout")
+        plan = _MOE_F32_PLANS[key] = (*out, L.vmoe_moe_f32_forward, L.vmoe_moe_f32_backward)
+    return plan
+
+
+class MoELayerOpF32(torch.autograd.Function):
+    """MoELayerOp for a float32 module (vmoe_moe_f32_forward / _backward): the
+    kernels, operands and order of router_topk, RoutedMoEOpF32 and RouterAuxOp,
+    so the same bits, in one call per direction. No routing-weight gradient.
+
+    forward(logits, x_flat, w1, w2, consts) as MoELayerOp's."""
+
+    @staticmethod
+    def forward(ctx, logits, x_flat, w1, w2, consts):
+        widths, ewo, coef, wn, top_k, block_size, max_width, normalize, _ = consts
+        T, d = x_flat.shape
+        E = widths.shape[0]
+        dev = x_flat.device
+        x_flat, w1, w2 = (_f32(x_flat, "TritonMoEMLP x"), _f32(w1, "TritonMoEMLP w1"),
+                          _f32(w2, "TritonMoEMLP w2"))
+        if not logits.is_contiguous() or logits.data_ptr() % 16:
+            logits = logits.clone(memory_format=torch.contiguous_format)
+        plan = _moe_f32_plan(T, E, top_k, block_size, d, max_width)
+        f32 = dict(dtype=torch.float32, device=dev)
+        saved = torch.empty(plan[0], dtype=torch.uint8, device=dev)
+        scratch = torch.empty(plan[1], dtype=torch.uint8, device=dev)
+        out = torch.empty(T, d, **f32)
+        losses = torch.empty(3, **f32)  # z, load balance, compute
+        f_i = torch.empty(E, **f32)
+        st = plan[3](logits.data_ptr(), T, E, top_k, int(bool(normalize)), block_size,
+                     x_flat.data_ptr(), x_flat.stride(0), w1.data_ptr(), w1.stride(0),
+                     w2.data_ptr(), w2.stride(0), ewo.data_ptr(), widths.data_ptr(), d, max_width,
+                     coef.data_ptr(), wn.data_ptr(), saved.data_ptr(), scratch.data_ptr(),
+                     out.data_ptr(), d, losses.data_ptr(), losses.data_ptr() + 4, f_i.data_ptr(),
+                     _lib.stream(dev))
+        if st != _lib.OK:
+            _lib.check(st, "vmoe_moe_f32_forward")
+        ctx.save_for_backward(logits, x_flat, w1, w2, saved)
+        ctx.consts = consts
+        ctx.mark_non_differentiable(f_i)
+        ctx.set_materialize_grads(False)  # as MoELayerOp
+        return out, losses[0], losses[1], losses[2], f_i
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_out, g_z, g_lb, g_cl, _g_fi):
+        logits, x_flat, w1, w2, saved = ctx.saved_tensors
+        widths, ewo, coef, wn, k, b, max_width, _, _ = ctx.consts
+        T, d = x_flat.shape
+        E = widths.shape[0]
+        dev = logits.device
+        plan = _moe_f32_plan(T, E, k, b, d, max_width)
+        gz, glb, gcl = _scalar_f32(g_z), _scalar_f32(g_lb), _scalar_f32(g_cl)
+        need = ctx.needs_input_grad
+        want_x = grad_out is not None and (need[1] or need[2] or need[3])
+        want_logits = need[0] and (gz is not None or glb is not None or gcl is not None)
+        if not want_x and not want_logits:
+            return None, None, None, None, None
+        grad_x = grad_w1 = grad_w2 = grad_logits = g = scratch = None
+        ldg = 0
+        if want_x:
+            g, ldg = _broadcast_rows(grad_out.to(torch.float32))
+            grad_x = torch.empty(T, d, dtype=torch.float32, device=dev)
+            grad_w1 = torch.empty(w1.shape, dtype=torch.float32, device=dev)
+            grad_w2 = torch.empty(w2.shape, dtype=torch.float32, device=dev)
+        if want_logits:
+            grad_logits = torch.empty(T, E, dtype=torch.float32, device=dev)
+        scratch = torch.empty(plan[2], dtype=torch.uint8, device=dev)
+        ptr = _lib.ptr
+        st = plan[4](saved.data_ptr(), logits.data_ptr(), T, E, k, b, x_flat.data_ptr(),
+                     x_flat.stride(0), w1.data_ptr(), w1.stride(0), w2.data_ptr(), w2.stride(0),
+                     ewo.data_ptr(), widths.data_ptr(), d, max_width, coef.data_ptr(),
+                     wn.data_ptr(), ptr(g), ldg, ptr(gz), ptr(glb), ptr(gcl), ptr(grad_x), d,
+                     ptr(grad_w1), w1.shape[1], ptr(grad_w2), d, ptr(grad_logits),
+                     scratch.data_ptr(), _lib.stream(dev))
+        if st != _lib.OK:
+            _lib.check(st, "vmoe_moe_f32_backward")
+        return grad_logits, grad_x, grad_w1, grad_w2, None
 
 
 class NoTokensOp(torch.autograd.Function):

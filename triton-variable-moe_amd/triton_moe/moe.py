@@ -39,7 +39,7 @@ from .kernels.fused_cumsum import route_device
 from .kernels.gather import combine_rows
 from .kernels import grouped_gemm as gg
 from .kernels.grouped_gemm import (CompactRoutedMoEOp, ExpertPathOp, GemmMeta, MoELayerOp,
-                                   MoERouterLayerOp, NoTokensOp,
+                                   MoELayerOpF32, MoERouterLayerOp, NoTokensOp,
                                    RoutedMoEOp, RoutedMoEOpF32, down_fwd, f32_down_fwd,
                                    f32_up_fwd, up_fwd)
 from .kernels.router import (RouterAuxOp, RouterLinear, RouterWeightOp, router_bwd_supported,
@@ -339,6 +339,17 @@ class TritonMoEMLP(nn.Module):
                 router_logits, x_flat, self.w1, self.w2, self._layer_consts(coef, wn))
             aux_loss = {"router_z_loss": z, "load_balance_loss": lb, "compute_loss": cl}
             return out.view(batch_size, seq_len, n_embd), aux_loss, f_i.to(x.dtype)
+        if (x_flat.shape[0] > 0 and router_logits.is_cuda and self.num_experts <= 2048 and
+                self.num_active_experts <= 64 and self.w1.dtype == torch.float32 and
+                self.w2.dtype == torch.float32 and x_flat.dtype == torch.float32 and
+                router_logits.dtype == torch.float32 and gg.FUSED_EXPERT_PATH and
+                _lib._launch_timer is None and
+                not (self.config.routing_weight_grad and torch.is_grad_enabled())):
+            coef, wn = self._aux_tables(router_logits.device)
+            out, z, lb, cl, f_i = MoELayerOpF32.apply(
+                router_logits, x_flat, self.w1, self.w2, self._layer_consts(coef, wn))
+            aux_loss = {"router_z_loss": z, "load_balance_loss": lb, "compute_loss": cl}
+            return out.view(batch_size, seq_len, n_embd), aux_loss, f_i
         state = router_topk(router_logits, self.num_active_experts, self.norm_topk_prob,
                             route_hist=True)
         weights = state.weights

@@ -868,3 +868,28 @@ def test_router_in_node_gradients(weight_grad, freeze, device):
     assert a[0] != b[0] or freeze in ("router", "x")  # the hooked router has a node of its own
     for u, v in zip(a[1:], b[1:]):
         assert (u is None) == (v is None) and (u is None or torch.equal(u, v))
+
+
+@pytest.mark.parametrize("E,T", [(72, 40), (128, 1531), (64, 300), (136, 200)])
+def test_losses_in_routing_launch_same_bits(E, T, device):
+    """The auxiliary losses formed beside the placement (both placement
+    kernels; 136 experts keep the launch of their own) carry the bits of the
+    per-kernel path, as do the output and the routing counts."""
+    from triton_moe.kernels import grouped_gemm as gg
+
+    torch.manual_seed(E)
+    cfg = TritonMoEConfig(n_embd=64, expert_sizes=[(E - 2, 64), (1, 128), (1, 64)],
+                          num_active_experts=4)
+    m = TritonMoEMLP(cfg).to(device).to(torch.bfloat16)
+    x = torch.randn(1, T, 64, device=device).to(torch.bfloat16)
+    got = []
+    for fused in (True, False):
+        gg.FUSED_EXPERT_PATH = fused
+        try:
+            with torch.no_grad():
+                out, aux, f_i = m(x)
+        finally:
+            gg.FUSED_EXPERT_PATH = True
+        got.append([out, f_i, *aux.values()])
+    for a, b in zip(*got):
+        assert bits_equal(a, b)

@@ -405,7 +405,8 @@ extern "C" int vmoe_moe_forward(const uint16_t* logits, int64_t num_tokens, int3
     VMOE_TRY(vmoe_router_topk(logits, E, num_tokens, E, top_k, normalize, wts, sel, nullptr,
                               nullptr, lse, partial, nfl, nullptr, stream));
   }
-  // The losses ride in the routing launch where it takes them (E <= 64),
+  // The losses ride in the routing launch where it takes them (one of the
+  // placement kernels that count for themselves, E <= 1024),
   // else they get their own launch after the expert path.
   const RouteAux aux = {partial, (int)M.partial_rows, num_tokens, coef, widths_normalized,
                         f_i, at<float>(saved, M.slot[VMOE_M_F_I32]),

@@ -1,6 +1,6 @@
 // The router's auxiliary-loss reduction as the device code of one 1024-thread
 // workgroup. router_aux_kernel (router.hip) runs it as a launch of its own;
-// route_small_kernel (route.hip) runs it in one extra workgroup beside the
+// route_small_kernel and route_fused_kernel (route.hip) run it in one extra workgroup beside the
 // routing placement when the MoE layer asks for it, so the layer's forward
 // has one launch fewer. Both run the same code with the same thread mapping,
 // so the losses carry the same bits either way.
@@ -120,7 +120,7 @@ __device__ __forceinline__ void router_aux_block(
   }
 }
 
-// Operands of the auxiliary losses for route_small_kernel's extra workgroup
+// Operands of the auxiliary losses for the placement kernels' extra workgroup
 // (the bf16 layer path, vmoe_moe_forward); partial == nullptr: no losses.
 struct RouteAux {
   const float* partial;  // [nblk][E + 1] of the top-k launch
@@ -136,7 +136,7 @@ struct RouteAux {
 };
 
 // vmoe_route_counted (route.hip) with the losses above folded into the
-// routing launch where the E <= 64 placement kernel runs: then *aux_done is
+// routing launch where one of those placement kernels runs: then *aux_done is
 // set and the caller skips its router_aux launch; otherwise *aux_done is
 // left false and nothing of `aux` is touched.
 int route_counted_aux(const void* sel, int32_t is64, int64_t A, int32_t E, int32_t top_k,

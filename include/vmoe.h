@@ -749,6 +749,23 @@ int vmoe_moe_backward(const void* saved, const uint16_t* logits, int64_t num_tok
                       void* scratch, void* dw_workspace, size_t dw_workspace_bytes,
                       vmoe_stream_t stream, vmoe_stream_t side_stream);
 
+/* vmoe_moe_backward and, where grad_logits is given, vmoe_router_linear_bwd on
+ * it for logits = x wr^T: grad_wr (nullable) and, with need_x, the token
+ * gradient added to the expert path's in grad_x (without grad_out: alone).
+ * router_workspace: vmoe_router_linear_bwd_workspace_bytes. */
+int vmoe_moe_router_backward(
+    const void* saved, const uint16_t* logits, int64_t num_tokens, int32_t num_experts,
+    int32_t top_k, int32_t normalize, int32_t block_size, const uint16_t* x, int64_t ldx,
+    const uint16_t* w1, int64_t ldw1, const uint16_t* w2, int64_t ldw2, const int32_t* ewo,
+    const int32_t* widths, int64_t hidden, int64_t max_width, const float* coef,
+    const float* widths_normalized, const uint16_t* grad_out, int64_t ldg,
+    const uint16_t* grad_scale, const float* grad_z, const float* grad_lb, const float* grad_cl,
+    int32_t weight_grad, uint16_t* grad_x, int64_t ldgx, uint16_t* grad_w1, int64_t ldgw1,
+    uint16_t* grad_w2, int64_t ldgw2, uint16_t* grad_logits, void* scratch, void* dw_workspace,
+    size_t dw_workspace_bytes, vmoe_stream_t stream, vmoe_stream_t side_stream,
+    const uint16_t* wr, int64_t ldwr, uint16_t* grad_wr, int64_t ldgwr, int32_t need_x,
+    void* router_workspace, size_t router_workspace_bytes);
+
 /* The float32 layer after its router Linear, one call per direction, as
  * vmoe_moe_forward / vmoe_moe_backward are for bf16: fp32 logits [T, E]
  * (contiguous; 16-byte aligned where E % 8 == 0), x, weights, losses and

@@ -833,16 +833,19 @@ def test_forward_without_autograd_same_bits(mode, device):
         assert bits_equal(aux[key], aux_g[key].detach()), key
 
 
-@pytest.mark.parametrize("weight_grad", [False, True])
+@pytest.mark.parametrize("weight_grad,E,k", [(False, 16, 3), (True, 16, 3), (False, 40, 2),
+                                             (False, 64, 8), (True, 72, 3), (False, 16, 9)])
 @pytest.mark.parametrize("freeze", ["none", "x", "router", "experts"])
-def test_router_in_node_gradients(weight_grad, freeze, device):
+def test_router_in_node_gradients(weight_grad, E, k, freeze, device):
     """The layer with its router Linear inside the autograd node against the
     same layer whose router has a (do-nothing) forward hook and therefore
     keeps its own linear node: outputs, losses and every gradient bit for bit
-    (the input's is a rounded product, then a rounded sum, on both)."""
+    (the input's is a rounded product, then a rounded sum, on both). With at
+    most 64 experts and 8 slots the node's launch also sums the expert path's
+    rows; 72 experts or 9 slots leave that to the combine."""
     torch.manual_seed(3)
-    cfg = TritonMoEConfig(n_embd=136, expert_sizes=[(4, 128), (12, 64)], num_active_experts=3,
-                          routing_weight_grad=weight_grad)
+    cfg = TritonMoEConfig(n_embd=136, expert_sizes=[(4, 128), (E - 4, 64)],
+                          num_active_experts=k, routing_weight_grad=weight_grad)
     m = TritonMoEMLP(cfg).to(device).to(torch.bfloat16)
     x = torch.randn(2, 331, 136, device=device).to(torch.bfloat16)
     g = torch.randn(2, 331, 136, device=device).to(torch.bfloat16)

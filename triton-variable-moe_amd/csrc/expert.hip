@@ -211,14 +211,20 @@ extern "C" int vmoe_expert_forward(const void* selected, int32_t selected_is_int
                         nullptr, nullptr);
 }
 
-extern "C" int vmoe_expert_backward(
+namespace vmoe {
+namespace {
+// vmoe_expert_backward; finish(gxg, rows, arow) turns the gathered dX rows into
+// grad_x on the main stream, beside the side stream's dW1.
+template <typename Finish>
+int expert_backward(
     const void* saved, int64_t num_tokens, int32_t num_experts, int32_t top_k,
     int32_t block_size, const uint16_t* x, int64_t ldx, const uint16_t* w1, int64_t ldw1,
     const uint16_t* w2, int64_t ldw2, const int32_t* ewo, const int32_t* widths, int64_t hidden,
     int64_t max_width, const uint16_t* grad_out, int64_t ldg, const uint16_t* grad_scale,
     uint16_t* grad_x, int64_t ldgx, uint16_t* grad_w1, int64_t ldgw1, uint16_t* grad_w2,
     int64_t ldgw2, uint16_t* grad_weights, void* scratch, void* dw_workspace,
-    size_t dw_workspace_bytes, vmoe_stream_t stream, vmoe_stream_t side_stream) {
+    size_t dw_workspace_bytes, vmoe_stream_t stream, vmoe_stream_t side_stream,
+    Finish&& finish) {
   Layout L;
   if (!make_layout(num_tokens, num_experts, top_k, block_size, hidden, max_width, true, L))
     return VMOE_ERR_INVALID_ARG;
@@ -280,9 +286,6 @@ extern "C" int vmoe_expert_backward(
     if (st == VMOE_OK) st = st2;
   }
   VMOE_TRY(st);
-  VMOE_TRY(vmoe_combine(gxg, L.cap, hidden, arow, nullptr, k, grad_x, ldgx, num_tokens, hidden,
-                        stream));
-  if (two) VMOE_TRY(order(main_s, side_s, ev[2]));
   if (grad_weights) {
     VMOE_TRY(vmoe_routing_weight_grad(row_dot, L.nblk, (int32_t)L.nblk, L.cap, rw, arow, L.A,
                                       grad_weights, stream));
@@ -290,7 +293,29 @@ extern "C" int vmoe_expert_backward(
                                              pre, max_width, rw, arow, L.A, k, eto, ewo, widths,
                                              E, hidden, L.cap, grad_weights, stream));
   }
+  VMOE_TRY(finish(gxg, L.cap, arow));
+  if (two) VMOE_TRY(order(main_s, side_s, ev[2]));
   return VMOE_OK;
+}
+}  // namespace
+}  // namespace vmoe
+
+extern "C" int vmoe_expert_backward(
+    const void* saved, int64_t num_tokens, int32_t num_experts, int32_t top_k,
+    int32_t block_size, const uint16_t* x, int64_t ldx, const uint16_t* w1, int64_t ldw1,
+    const uint16_t* w2, int64_t ldw2, const int32_t* ewo, const int32_t* widths, int64_t hidden,
+    int64_t max_width, const uint16_t* grad_out, int64_t ldg, const uint16_t* grad_scale,
+    uint16_t* grad_x, int64_t ldgx, uint16_t* grad_w1, int64_t ldgw1, uint16_t* grad_w2,
+    int64_t ldgw2, uint16_t* grad_weights, void* scratch, void* dw_workspace,
+    size_t dw_workspace_bytes, vmoe_stream_t stream, vmoe_stream_t side_stream) {
+  return expert_backward(
+      saved, num_tokens, num_experts, top_k, block_size, x, ldx, w1, ldw1, w2, ldw2, ewo, widths,
+      hidden, max_width, grad_out, ldg, grad_scale, grad_x, ldgx, grad_w1, ldgw1, grad_w2, ldgw2,
+      grad_weights, scratch, dw_workspace, dw_workspace_bytes, stream, side_stream,
+      [&](const uint16_t* gxg, int64_t rows, const int32_t* arow) {
+        return vmoe_combine(gxg, rows, hidden, arow, nullptr, top_k, grad_x, ldgx, num_tokens,
+                            hidden, stream);
+      });
 }
 
 // ---------------------------------------------------------------------------
@@ -423,6 +448,94 @@ extern "C" int vmoe_moe_forward(const uint16_t* logits, int64_t num_tokens, int3
                          z_loss, losses, stream);
 }
 
+namespace vmoe {
+namespace {
+// The router Linear's share of vmoe_moe_router_backward.
+struct RouterGrad {
+  const uint16_t* wr;
+  int64_t ldwr;
+  uint16_t* grad_wr;  // nullable
+  int64_t ldgwr;
+  bool need_x;
+  void* ws;
+  size_t ws_bytes;
+};
+
+int moe_backward(
+    const void* saved, const uint16_t* logits, int64_t num_tokens, int32_t num_experts,
+    int32_t top_k, int32_t normalize, int32_t block_size, const uint16_t* x, int64_t ldx,
+    const uint16_t* w1, int64_t ldw1, const uint16_t* w2, int64_t ldw2, const int32_t* ewo,
+    const int32_t* widths, int64_t hidden, int64_t max_width, const float* coef,
+    const float* widths_normalized, const uint16_t* grad_out, int64_t ldg,
+    const uint16_t* grad_scale, const float* grad_z, const float* grad_lb, const float* grad_cl,
+    int32_t weight_grad, uint16_t* grad_x, int64_t ldgx, uint16_t* grad_w1, int64_t ldgw1,
+    uint16_t* grad_w2, int64_t ldgw2, uint16_t* grad_logits, void* scratch, void* dw_workspace,
+    size_t dw_workspace_bytes, vmoe_stream_t stream, vmoe_stream_t side_stream,
+    const RouterGrad* router) {
+  MoeLayout M;
+  if (!make_moe_layout(num_tokens, num_experts, top_k, block_size, hidden, max_width, M))
+    return VMOE_ERR_INVALID_ARG;
+  if (num_tokens == 0) return VMOE_OK;
+  if (!saved || !scratch) return VMOE_ERR_INVALID_ARG;
+  const int E = num_experts;
+  const int64_t T = num_tokens;
+  uint16_t* gw = weight_grad && grad_out && grad_logits ? at<uint16_t>(scratch, M.b_gw) : nullptr;
+  const bool aux = grad_z || grad_lb || grad_cl;
+  if (grad_logits) {
+    if (!aux && !gw) return VMOE_ERR_INVALID_ARG;  // the caller returns no logit gradient then
+    if (!logits || !coef || !widths_normalized) return VMOE_ERR_INVALID_ARG;
+  }
+  auto logit_grad = [&]() -> int {
+    const float* lse = at<float>(saved, M.slot[VMOE_M_LSE]);
+    const float* f_i32 = at<float>(saved, M.slot[VMOE_M_F_I32]);
+    if (aux)
+      VMOE_TRY(vmoe_router_aux_bwd(logits, E, T, E, lse, f_i32, coef, widths_normalized, grad_z,
+                                   grad_lb, grad_cl, grad_logits, E, stream));
+    if (gw) {
+      uint16_t* dst = aux ? at<uint16_t>(scratch, M.b_gl) : grad_logits;
+      VMOE_TRY(vmoe_router_weight_bwd(logits, E, T, E, top_k, normalize,
+                                      at<int32_t>(saved, M.slot[VMOE_M_SELECTED]), nullptr, gw,
+                                      top_k, dst, E, stream));
+      if (aux) {
+        const int64_t n = T * E;
+        VMOE_LAUNCH(add_bf16_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)),
+                    dim3(256), 0, reinterpret_cast<hipStream_t>(stream), grad_logits, dst, n);
+        VMOE_CHECK_LAUNCH();
+      }
+    }
+    return VMOE_OK;
+  };
+  // With the router's gradients in the same call, grad_x is formed where they
+  // are: one launch reads the dX rows and writes grad_x once.
+  const bool fused = router && router->need_x && grad_logits && grad_out &&
+                     top_k <= kRowSumSlots && E <= kRowSumExperts;
+  auto router_grad = [&](const RowSum* sum) {
+    return router_linear_bwd(grad_logits, x, ldx, router->wr, router->ldwr, T, hidden, E,
+                             router->need_x ? grad_x : nullptr, ldgx, grad_out != nullptr,
+                             router->grad_wr, router->ldgwr, router->ws, router->ws_bytes, sum,
+                             stream);
+  };
+  if (grad_out) {
+    VMOE_TRY(expert_backward(
+        saved, T, E, top_k, block_size, x, ldx, w1, ldw1, w2, ldw2, ewo, widths, hidden, max_width,
+        grad_out, ldg, grad_scale, grad_x, ldgx, grad_w1, ldgw1, grad_w2, ldgw2, gw, scratch,
+        dw_workspace, dw_workspace_bytes, stream, side_stream,
+        [&](const uint16_t* gxg, int64_t rows, const int32_t* arow) -> int {
+          if (!fused)
+            return vmoe_combine(gxg, rows, hidden, arow, nullptr, top_k, grad_x, ldgx, T, hidden,
+                                stream);
+          VMOE_TRY(logit_grad());
+          const RowSum sum = {gxg, hidden, rows, arow, top_k};
+          return router_grad(&sum);
+        }));
+  }
+  if (!grad_logits || fused) return VMOE_OK;
+  VMOE_TRY(logit_grad());
+  return router ? router_grad(nullptr) : VMOE_OK;
+}
+}  // namespace
+}  // namespace vmoe
+
 extern "C" int vmoe_moe_backward(
     const void* saved, const uint16_t* logits, int64_t num_tokens, int32_t num_experts,
     int32_t top_k, int32_t normalize, int32_t block_size, const uint16_t* x, int64_t ldx,
@@ -433,40 +546,28 @@ extern "C" int vmoe_moe_backward(
     int32_t weight_grad, uint16_t* grad_x, int64_t ldgx, uint16_t* grad_w1, int64_t ldgw1,
     uint16_t* grad_w2, int64_t ldgw2, uint16_t* grad_logits, void* scratch, void* dw_workspace,
     size_t dw_workspace_bytes, vmoe_stream_t stream, vmoe_stream_t side_stream) {
-  MoeLayout M;
-  if (!make_moe_layout(num_tokens, num_experts, top_k, block_size, hidden, max_width, M))
-    return VMOE_ERR_INVALID_ARG;
-  if (num_tokens == 0) return VMOE_OK;
-  if (!saved || !scratch) return VMOE_ERR_INVALID_ARG;
-  const int E = num_experts;
-  const int64_t T = num_tokens;
-  uint16_t* gw = weight_grad && grad_out && grad_logits ? at<uint16_t>(scratch, M.b_gw) : nullptr;
-  if (grad_out) {
-    VMOE_TRY(vmoe_expert_backward(saved, T, E, top_k, block_size, x, ldx, w1, ldw1, w2, ldw2, ewo,
-                                  widths, hidden, max_width, grad_out, ldg, grad_scale, grad_x,
-                                  ldgx, grad_w1, ldgw1, grad_w2, ldgw2, gw, scratch, dw_workspace,
-                                  dw_workspace_bytes, stream, side_stream));
-  }
-  if (!grad_logits) return VMOE_OK;
-  const bool aux = grad_z || grad_lb || grad_cl;
-  if (!aux && !gw) return VMOE_ERR_INVALID_ARG;  // the caller returns no logit gradient then
-  if (!logits || !coef || !widths_normalized) return VMOE_ERR_INVALID_ARG;
-  const float* lse = at<float>(saved, M.slot[VMOE_M_LSE]);
-  const float* f_i32 = at<float>(saved, M.slot[VMOE_M_F_I32]);
-  if (aux)
-    VMOE_TRY(vmoe_router_aux_bwd(logits, E, T, E, lse, f_i32, coef, widths_normalized, grad_z,
-                                 grad_lb, grad_cl, grad_logits, E, stream));
-  if (gw) {
-    uint16_t* dst = aux ? at<uint16_t>(scratch, M.b_gl) : grad_logits;
-    VMOE_TRY(vmoe_router_weight_bwd(logits, E, T, E, top_k, normalize,
-                                    at<int32_t>(saved, M.slot[VMOE_M_SELECTED]), nullptr, gw,
-                                    top_k, dst, E, stream));
-    if (aux) {
-      const int64_t n = T * E;
-      VMOE_LAUNCH(add_bf16_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)),
-                         dim3(256), 0, reinterpret_cast<hipStream_t>(stream), grad_logits, dst, n);
-      VMOE_CHECK_LAUNCH();
-    }
-  }
-  return VMOE_OK;
+  return moe_backward(saved, logits, num_tokens, num_experts, top_k, normalize, block_size, x, ldx, w1, ldw1, w2,
+      ldw2, ewo, widths, hidden, max_width, coef, widths_normalized, grad_out, ldg, grad_scale, grad_z,
+      grad_lb, grad_cl, weight_grad, grad_x, ldgx, grad_w1, ldgw1, grad_w2, ldgw2, grad_logits,
+      scratch, dw_workspace, dw_workspace_bytes, stream, side_stream, nullptr);
+}
+
+extern "C" int vmoe_moe_router_backward(
+    const void* saved, const uint16_t* logits, int64_t num_tokens, int32_t num_experts,
+    int32_t top_k, int32_t normalize, int32_t block_size, const uint16_t* x, int64_t ldx,
+    const uint16_t* w1, int64_t ldw1, const uint16_t* w2, int64_t ldw2, const int32_t* ewo,
+    const int32_t* widths, int64_t hidden, int64_t max_width, const float* coef,
+    const float* widths_normalized, const uint16_t* grad_out, int64_t ldg,
+    const uint16_t* grad_scale, const float* grad_z, const float* grad_lb, const float* grad_cl,
+    int32_t weight_grad, uint16_t* grad_x, int64_t ldgx, uint16_t* grad_w1, int64_t ldgw1,
+    uint16_t* grad_w2, int64_t ldgw2, uint16_t* grad_logits, void* scratch, void* dw_workspace,
+    size_t dw_workspace_bytes, vmoe_stream_t stream, vmoe_stream_t side_stream,
+    const uint16_t* wr, int64_t ldwr, uint16_t* grad_wr, int64_t ldgwr, int32_t need_x,
+    void* router_workspace, size_t router_workspace_bytes) {
+  const RouterGrad router = {wr, ldwr, grad_wr, ldgwr, need_x != 0, router_workspace,
+                             router_workspace_bytes};
+  return moe_backward(saved, logits, num_tokens, num_experts, top_k, normalize, block_size, x, ldx, w1, ldw1, w2,
+      ldw2, ewo, widths, hidden, max_width, coef, widths_normalized, grad_out, ldg, grad_scale, grad_z,
+      grad_lb, grad_cl, weight_grad, grad_x, ldgx, grad_w1, ldgw1, grad_w2, ldgw2, grad_logits,
+      scratch, dw_workspace, dw_workspace_bytes, stream, side_stream, &router);
 }

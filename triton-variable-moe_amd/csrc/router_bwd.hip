@@ -67,6 +67,12 @@ struct RbArgs {
   int64_t T;
   int E, d, slabs, chunks, per, add;  // per: tokens per chunk
   int iters;  // grad_x: 128-token steps per workgroup
+  // what grad_x is added to, instead of its old values: the combine of the
+  // expert path's gradient rows, sum_j y[arow[t k + j]] (vmoe_combine)
+  const uint16_t* y;
+  int64_t ldy, y_rows;
+  const int32_t* arow;
+  int k;
 };
 
 // grad_w of columns [c0, c0 + 128) over the tokens of one chunk: stages of 128
@@ -151,6 +157,46 @@ __device__ __forceinline__ void rb_grad_w(const RbArgs& p, int block, char* lds)
     }
 }
 
+// The combine of 2 x 8 tokens' rows for 8 of the wave's columns per lane (8
+// lanes to a token): every slot's 16 bytes are in flight before any is summed,
+// the sum runs in slot order in fp32 and is rounded once, as in
+// combine_k_kernel. idx: the lane's token's row for slot lane % 8 of each.
+template <int KMAX>
+__device__ __forceinline__ void rb_combine(const RbArgs& p, const int32_t (&idx)[2], int col,
+                                           rb_u32x4 (&out)[2]) {
+  const int lane = threadIdx.x & 63;
+  rb_u32x4 v[2][KMAX];
+  bool ok[2][KMAX];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {
+      const int32_t row = __shfl(idx[u], (lane & 56) + j, kWave);
+      ok[u][j] = row >= 0 && col < p.d;
+      const rb_u32x4 z = {0, 0, 0, 0};
+      v[u][j] = ok[u][j] ? __builtin_nontemporal_load(reinterpret_cast<const rb_u32x4*>(
+                               p.y + (int64_t)row * p.ldy + col))
+                         : z;
+    }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    float acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j)
+      if (ok[u][j]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          acc[2 * q] += lo_f32(v[u][j][q]);
+          acc[2 * q + 1] += hi_f32(v[u][j][q]);
+        }
+      }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) out[u][q] = pack_bf16(acc[2 * q], acc[2 * q + 1]);
+  }
+}
+
 // grad_x of 128 * p.iters tokens x 128 columns, 32 tokens per wave and step:
 // w's columns stay in LDS (transposing reads), each wave reads its own gradient
 // rows straight from memory as fragments, and its fp32 results go through a
@@ -160,7 +206,13 @@ __device__ __forceinline__ void rb_grad_w(const RbArgs& p, int block, char* lds)
 // gradient rows, and one step per workgroup reads w's columns, 32 KB at
 // E = 128, for every 16 KB of grad_x: 108 and 130 us at 32768 x 2048,
 // E = 128, against 60 here and 52 for its bytes.)
-template <int MB>
+// KMAX > 0: the sum of the expert path's rows (at most KMAX per token) is formed
+// here instead of by a combine launch that writes grad_x for this one to read
+// back (combine and this launch, then this launch alone: 52 + 29 -> 74 us at
+// 16384 x 1024, E = 64, k = 8; 15 + 19 -> 23 us at 16384 x 768, E = 16, k = 2).
+// Up to 64 experts: at 128 the larger tile of w leaves fewer workgroups per CU
+// for the row reads (32768 x 2048, k = 8: 213 + 107 against 323 us).
+template <int MB, int KMAX>
 __device__ __forceinline__ void rb_grad_x(const RbArgs& p, int block, char* lds) {
   rb_lds* ws = (rb_lds*)lds;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -191,16 +243,37 @@ __device__ __forceinline__ void rb_grad_x(const RbArgs& p, int block, char* lds)
           t < p.T && k < p.E ? *reinterpret_cast<const rb_u32x4*>(p.g + t * p.E + k) : z);
     }
     rb_u32x4 old[2][4];  // (64-column half, 8 rows each)
-#pragma unroll
-    for (int hf = 0; hf < 2; ++hf)
+    if constexpr (KMAX > 0) {
+      int32_t idx[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int64_t t = t0 + 8 * i + (lane >> 3);
-        const int col = c0 + 64 * hf + (lane & 7) * 8;
-        const rb_u32x4 z = {0, 0, 0, 0};
-        old[hf][i] = p.add && t < p.T && col < p.d
-                         ? *reinterpret_cast<const rb_u32x4*>(p.gx + t * p.ldgx + col) : z;
+        const int32_t row =
+            t < p.T && (lane & 7) < p.k ? p.arow[t * p.k + (lane & 7)] : -1;
+        idx[i] = row < p.y_rows ? row : -1;
       }
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          const int32_t two[2] = {idx[i], idx[i + 1]};
+          rb_u32x4 sum[2];
+          rb_combine<KMAX>(p, two, c0 + 64 * hf + (lane & 7) * 8, sum);
+          old[hf][i] = sum[0];
+          old[hf][i + 1] = sum[1];
+        }
+    } else {
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int64_t t = t0 + 8 * i + (lane >> 3);
+          const int col = c0 + 64 * hf + (lane & 7) * 8;
+          const rb_u32x4 z = {0, 0, 0, 0};
+          old[hf][i] = p.add && t < p.T && col < p.d
+                           ? *reinterpret_cast<const rb_u32x4*>(p.gx + t * p.ldgx + col) : z;
+        }
+    }
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
       rb_f32x16 acc[2];
@@ -234,21 +307,22 @@ __device__ __forceinline__ void rb_grad_x(const RbArgs& p, int block, char* lds)
         // gradient added to the other one's by autograd
         rb_u32x4 res = {pack_bf16(u.x, u.y), pack_bf16(u.z, u.w), pack_bf16(v.x, v.y),
                         pack_bf16(v.z, v.w)};
-        if (p.add) {
+        if (KMAX > 0 || p.add) {
           const rb_u32x4 o = old[hf][i];
 #pragma unroll
           for (int q = 0; q < 4; ++q)
             res[q] = pack_bf16(lo_f32(o[q]) + lo_f32(res[q]), hi_f32(o[q]) + hi_f32(res[q]));
         }
         if (t0 + r < p.T && c0 + cc < p.d)
-          *reinterpret_cast<rb_u32x4*>(p.gx + (t0 + r) * p.ldgx + c0 + cc) = res;
+          __builtin_nontemporal_store(
+              res, reinterpret_cast<rb_u32x4*>(p.gx + (t0 + r) * p.ldgx + c0 + cc));
       }
       __builtin_amdgcn_wave_barrier();
     }
   }
 }
 
-template <int MB>
+template <int MB, int KMAX>
 __global__ __launch_bounds__(kRbThreads) void router_linear_bwd_kernel(RbArgs p) {
   constexpr int DW = kRbTokens * (kRbXStride + rb_gstride(MB));
   constexpr int DX = 32 * MB * kRbXStride + kRbRows * kRbOutStride * 4;
@@ -257,7 +331,7 @@ __global__ __launch_bounds__(kRbThreads) void router_linear_bwd_kernel(RbArgs p)
   if ((int)blockIdx.x < ndw)
     rb_grad_w<MB>(p, blockIdx.x, lds);
   else
-    rb_grad_x<MB>(p, blockIdx.x - ndw, lds);
+    rb_grad_x<MB, KMAX>(p, blockIdx.x - ndw, lds);
 }
 
 // grad_w = bf16(sum over the chunks, in order), four columns per thread.
@@ -307,12 +381,12 @@ extern "C" size_t vmoe_router_linear_bwd_workspace_bytes(int64_t num_tokens, int
   return chunks > 1 ? (size_t)chunks * (size_t)num_experts * (size_t)hidden * sizeof(float) : 0;
 }
 
-extern "C" int vmoe_router_linear_bwd(const uint16_t* grad_logits, const uint16_t* x, int64_t ldx,
-                                      const uint16_t* weight, int64_t ldw, int64_t num_tokens,
-                                      int64_t hidden, int32_t num_experts, uint16_t* grad_x,
-                                      int64_t ldgx, int32_t accumulate, uint16_t* grad_weight,
-                                      int64_t ldgw, void* workspace, size_t workspace_bytes,
-                                      vmoe_stream_t stream) {
+namespace vmoe {
+int router_linear_bwd(const uint16_t* grad_logits, const uint16_t* x, int64_t ldx,
+                      const uint16_t* weight, int64_t ldw, int64_t num_tokens, int64_t hidden,
+                      int32_t num_experts, uint16_t* grad_x, int64_t ldgx, int32_t accumulate,
+                      uint16_t* grad_weight, int64_t ldgw, void* workspace,
+                      size_t workspace_bytes, const RowSum* sum, vmoe_stream_t stream) {
   if (num_tokens < 0 || hidden <= 0 || num_experts <= 0) return VMOE_ERR_INVALID_ARG;
   if (!grad_x && !grad_weight) return VMOE_OK;
   if (num_tokens == 0) return VMOE_ERR_INVALID_ARG;  // grad_weight would be left unwritten
@@ -334,6 +408,13 @@ extern "C" int vmoe_router_linear_bwd(const uint16_t* grad_logits, const uint16_
   p.gx = grad_x; p.ldgx = ldgx; p.add = accumulate != 0;
   p.gw = grad_weight; p.ldgw = ldgw;
   p.T = num_tokens; p.E = num_experts; p.d = (int)hidden;
+  int kmax = 0;
+  if (grad_x && sum) {
+    if (!sum->y || !sum->arow || sum->k <= 0 || sum->ldy < hidden) return VMOE_ERR_INVALID_ARG;
+    if (sum->k > kRowSumSlots || num_experts > kRowSumExperts || sum->ldy % 8 != 0 || !a16(sum->y)) return VMOE_ERR_UNSUPPORTED;
+    p.y = sum->y; p.ldy = sum->ldy; p.y_rows = sum->rows; p.arow = sum->arow; p.k = sum->k;
+    kmax = sum->k <= 2 ? 2 : 8;
+  }
   rb_split(num_tokens, hidden, p.slabs, p.chunks, p.per);
   if (grad_weight && p.chunks > 1) {
     if (workspace_bytes < vmoe_router_linear_bwd_workspace_bytes(num_tokens, hidden, num_experts) ||
@@ -349,11 +430,21 @@ extern "C" int vmoe_router_linear_bwd(const uint16_t* grad_logits, const uint16_
   if (blocks > INT32_MAX) return VMOE_ERR_UNSUPPORTED;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)blocks), wg(kRbThreads);
-  switch ((num_experts + 31) / 32) {
-    case 1: VMOE_LAUNCH(router_linear_bwd_kernel<1>, grid, wg, 0, s, p); break;
-    case 2: VMOE_LAUNCH(router_linear_bwd_kernel<2>, grid, wg, 0, s, p); break;
-    case 3: VMOE_LAUNCH(router_linear_bwd_kernel<3>, grid, wg, 0, s, p); break;
-    default: VMOE_LAUNCH(router_linear_bwd_kernel<4>, grid, wg, 0, s, p); break;
+  switch ((num_experts + 31) / 32 * 16 + kmax) {
+#define VMOE_RB_CASE(M, K)                                                        \
+  case M * 16 + K:                                                                \
+    VMOE_LAUNCH((router_linear_bwd_kernel<M, K>), grid, wg, 0, s, p);             \
+    break;
+    VMOE_RB_CASE(1, 0)
+    VMOE_RB_CASE(1, 2)
+    VMOE_RB_CASE(1, 8)
+    VMOE_RB_CASE(2, 0)
+    VMOE_RB_CASE(2, 2)
+    VMOE_RB_CASE(2, 8)
+    VMOE_RB_CASE(3, 0)
+    VMOE_RB_CASE(4, 0)
+#undef VMOE_RB_CASE
+    default: return VMOE_ERR_UNSUPPORTED;
   }
   VMOE_CHECK_LAUNCH();
   if (grad_weight && p.chunks > 1) {
@@ -363,4 +454,16 @@ extern "C" int vmoe_router_linear_bwd(const uint16_t* grad_logits, const uint16_
     VMOE_CHECK_LAUNCH();
   }
   return VMOE_OK;
+}
+}  // namespace vmoe
+
+extern "C" int vmoe_router_linear_bwd(const uint16_t* grad_logits, const uint16_t* x, int64_t ldx,
+                                      const uint16_t* weight, int64_t ldw, int64_t num_tokens,
+                                      int64_t hidden, int32_t num_experts, uint16_t* grad_x,
+                                      int64_t ldgx, int32_t accumulate, uint16_t* grad_weight,
+                                      int64_t ldgw, void* workspace, size_t workspace_bytes,
+                                      vmoe_stream_t stream) {
+  return router_linear_bwd(grad_logits, x, ldx, weight, ldw, num_tokens, hidden, num_experts,
+                           grad_x, ldgx, accumulate, grad_weight, ldgw, workspace,
+                           workspace_bytes, nullptr, stream);
 }

@@ -35,6 +35,23 @@ extern thread_local LaunchTiming g_launch_timing;
 void gemm_pair_begin();
 int gemm_pair_end();
 
+// router_bwd.hip: vmoe_router_linear_bwd; with `sum`, grad_x's starting values
+// are the unweighted combine of `rows` rows y through arow (vmoe_combine's
+// values) instead of its old ones, for k <= kRowSumSlots slots per token and at
+// most kRowSumExperts experts.
+constexpr int kRowSumSlots = 8, kRowSumExperts = 64;
+struct RowSum {
+  const uint16_t* y;
+  int64_t ldy, rows;
+  const int32_t* arow;
+  int32_t k;
+};
+int router_linear_bwd(const uint16_t* grad_logits, const uint16_t* x, int64_t ldx,
+                      const uint16_t* weight, int64_t ldw, int64_t num_tokens, int64_t hidden,
+                      int32_t num_experts, uint16_t* grad_x, int64_t ldgx, int32_t accumulate,
+                      uint16_t* grad_weight, int64_t ldgw, void* workspace,
+                      size_t workspace_bytes, const RowSum* sum, vmoe_stream_t stream);
+
 // gemm_f32.hip: vmoe_gemm_f32_down_bwd_dh with the relu^2 rule in the epilogue,
 // ga = pre > 0 ? 2 gh pre : 0 for gh = grad_y W2_e^T (pre and ga share ldga):
 // the values vmoe_f32_relu2_grad forms from a stored gh.

@@ -30,7 +30,6 @@ from torch.autograd.function import once_differentiable
 
 from .. import _lib
 from .gather import _broadcast_rows, row_maps
-from .router import router_bwd
 
 _ACTIVATIONS = {"none": _lib.ACT_NONE, "relu_squared": _lib.ACT_RELU_SQUARED}
 
@@ -1127,7 +1126,8 @@ def _moe_plan(T: int, E: int, k: int, block_size: int, hidden: int, max_width: i
     """Everything MoELayerOp's two calls need that depends on the shape only,
     looked up once: (saved_bytes, fwd_scratch_bytes, bwd_scratch_bytes,
     rows_bound, dW workspace bytes, side stream by size, the ones row of
-    out.sum()'s gradient, the two library functions). An eager step at cfg1
+    out.sum()'s gradient, the two library functions, the router gradient's
+    workspace bytes and the backward that includes it). An eager step at cfg1
     is host-bound, so per-step Python is step time."""
     key = (T, E, k, block_size, hidden, max_width, device.index)
     plan = _MOE_PLANS.get(key)
@@ -1138,7 +1138,9 @@ def _moe_plan(T: int, E: int, k: int, block_size: int, hidden: int, max_width: i
         plan = _MOE_PLANS[key] = (
             saved_b, fwd_b, bwd_b, rows, ws_n,
             T * k * max_width * hidden >= SIDE_STREAM_MIN_WORK, _ones_row(hidden, device),
-            _lib.lib().vmoe_moe_forward, _lib.lib().vmoe_moe_backward)
+            _lib.lib().vmoe_moe_forward, _lib.lib().vmoe_moe_backward,
+            int(_lib.lib().vmoe_router_linear_bwd_workspace_bytes(T, hidden, E)),
+            _lib.lib().vmoe_moe_router_backward)
     return plan
 
 
@@ -1172,8 +1174,8 @@ class MoELayerOp(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, grad_out, g_z, g_lb, g_cl, _g_fi):
         need = ctx.needs_input_grad
-        grad_logits, grad_x, grad_w1, grad_w2 = _moe_backward(
-            ctx, grad_out, g_z, g_lb, g_cl, need[0], need[1] or need[2] or need[3])
+        grad_logits, grad_x, grad_w1, grad_w2, _ = _moe_backward(
+            ctx, grad_out, g_z, g_lb, g_cl, need[0], need[1] or need[2] or need[3], None)
         return grad_logits, grad_x, grad_w1, grad_w2, None
 
 
@@ -1193,12 +1195,9 @@ class MoERouterLayerOp(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, grad_out, g_z, g_lb, g_cl, _g_fi):
         need_x, need_wr, need_w1, need_w2, _ = ctx.needs_input_grad
-        grad_logits, grad_x, grad_w1, grad_w2 = _moe_backward(
-            ctx, grad_out, g_z, g_lb, g_cl, need_x or need_wr, need_x or need_w1 or need_w2)
-        grad_wr = None
-        if grad_logits is not None:
-            grad_x, grad_wr = router_bwd(grad_logits, ctx.saved_tensors[1], ctx.saved_tensors[5],
-                                         need_x, need_wr, grad_x)
+        _, grad_x, grad_w1, grad_w2, grad_wr = _moe_backward(
+            ctx, grad_out, g_z, g_lb, g_cl, need_x or need_wr, need_x or need_w1 or need_w2,
+            (need_x, need_wr))
         return grad_x, grad_wr, grad_w1, grad_w2, None
 
 
@@ -1238,8 +1237,10 @@ def _moe_forward(ctx, logits, x_flat, w1, w2, wr, consts):
     return out, z, losses[0], losses[1], f_i
 
 
-def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts):
-    """(grad_logits, grad_x, grad_w1, grad_w2), None where not formed."""
+def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts, router):
+    """(grad_logits, grad_x, grad_w1, grad_w2, grad_wr), None where not formed.
+    router: (whether x, whether the router weight needs a gradient) of a node
+    that holds the router Linear (vmoe_moe_router_backward), else None."""
     logits, x_flat, w1, w2, saved = ctx.saved_tensors[:5]
     widths, ewo, coef, wn, k, b, max_width, _, weight_grad = ctx.consts
     T, E, d, norm = ctx.dims
@@ -1266,7 +1267,7 @@ def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts):
     if want_logits:
         grad_logits = torch.empty(T, E, dtype=torch.bfloat16, device=dev)
     if not want_x and not want_logits:
-        return None, None, None, None
+        return None, None, None, None, None
     scratch = torch.empty(plan[2], dtype=torch.uint8, device=dev)
     main = _lib.stream(dev)
     use_side = BACKWARD_SIDE_STREAM if BACKWARD_SIDE_STREAM is not None else plan[5]
@@ -1276,16 +1277,30 @@ def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts):
     if ws is None or ws.numel() < plan[4]:
         ws = _dw_workspace_bytes(E, d, max_width, plan[3], dev, ws_stream)
     ptr = _lib.ptr
-    st = plan[8](saved.data_ptr(), logits.data_ptr(), T, E, k, norm, b,
-                 x_flat.data_ptr(), x_flat.stride(0), w1.data_ptr(), w1.stride(0),
-                 w2.data_ptr(), w2.stride(0), ewo.data_ptr(), widths.data_ptr(), d, max_width,
-                 coef.data_ptr(), wn.data_ptr(), ptr(g), ldg, ptr(gs), ptr(gz), ptr(glb),
-                 ptr(gcl), int(bool(weight_grad)), ptr(grad_x), d, ptr(grad_w1), w1.stride(0),
-                 ptr(grad_w2), w2.stride(0), ptr(grad_logits), scratch.data_ptr(),
-                 ws.data_ptr(), ws.numel(), main, side)
+    grad_wr = None
+    extra = ()
+    if router is not None and want_logits:
+        need_x, need_wr = router
+        wr = ctx.saved_tensors[5]
+        if need_x and grad_x is None:
+            grad_x = torch.empty(T, d, dtype=torch.bfloat16, device=dev)
+        n = 0
+        rws = None
+        if need_wr:
+            grad_wr = torch.empty(E, d, dtype=torch.bfloat16, device=dev)
+            n = plan[9]
+            rws = torch.empty(n, dtype=torch.uint8, device=dev) if n else None
+        extra = (wr.data_ptr(), wr.stride(0), ptr(grad_wr), d, int(need_x), ptr(rws), n)
+    st = plan[10 if extra else 8](
+        saved.data_ptr(), logits.data_ptr(), T, E, k, norm, b, x_flat.data_ptr(),
+        x_flat.stride(0), w1.data_ptr(), w1.stride(0), w2.data_ptr(), w2.stride(0),
+        ewo.data_ptr(), widths.data_ptr(), d, max_width, coef.data_ptr(), wn.data_ptr(), ptr(g),
+        ldg, ptr(gs), ptr(gz), ptr(glb), ptr(gcl), int(bool(weight_grad)), ptr(grad_x), d,
+        ptr(grad_w1), w1.stride(0), ptr(grad_w2), w2.stride(0), ptr(grad_logits),
+        scratch.data_ptr(), ws.data_ptr(), ws.numel(), main, side, *extra)
     if st != _lib.OK:
-        _lib.check(st, "vmoe_moe_backward")
-    return grad_logits, grad_x, grad_w1, grad_w2
+        _lib.check(st, "vmoe_moe_router_backward" if extra else "vmoe_moe_backward")
+    return grad_logits, grad_x, grad_w1, grad_w2, grad_wr
 
 
 def _scalar_f32(g):

@@ -143,22 +143,19 @@ def router_bwd_supported(wr: torch.Tensor) -> bool:
             wr.stride(0) >= d and wr.data_ptr() % 16 == 0)
 
 
-def router_bwd(g: torch.Tensor, x2d: torch.Tensor, wr: torch.Tensor, need_x: bool, need_w: bool,
-               grad_x: torch.Tensor | None = None):
+def router_bwd(g: torch.Tensor, x2d: torch.Tensor, wr: torch.Tensor, need_x: bool, need_w: bool):
     """(grad_x, grad_w) of the router Linear from contiguous logit gradients g
-    [T, E] (vmoe_router_linear_bwd); a grad_x given is added to in place."""
+    [T, E] (vmoe_router_linear_bwd), None where not needed."""
     T, d = x2d.shape
     E = wr.shape[0]
     dev = g.device
-    add = grad_x is not None
-    if need_x and not add:
-        grad_x = torch.empty(T, d, dtype=torch.bfloat16, device=dev)
+    grad_x = torch.empty(T, d, dtype=torch.bfloat16, device=dev) if need_x else None
     grad_w = torch.empty(E, d, dtype=torch.bfloat16, device=dev) if need_w else None
     n = int(_lib.lib().vmoe_router_linear_bwd_workspace_bytes(T, d, E)) if need_w else 0
     ws = torch.empty(n, dtype=torch.uint8, device=dev) if n else None
     _lib.call("vmoe_router_linear_bwd", g.data_ptr(), x2d.data_ptr(), x2d.stride(0),
-              wr.data_ptr(), wr.stride(0), T, d, E, grad_x.data_ptr() if need_x else None, d,
-              int(add), _lib.ptr(grad_w), d, _lib.ptr(ws), n, _lib.stream(dev))
+              wr.data_ptr(), wr.stride(0), T, d, E, _lib.ptr(grad_x), d, 0, _lib.ptr(grad_w), d,
+              _lib.ptr(ws), n, _lib.stream(dev))
     return grad_x, grad_w
 
 

@@ -722,8 +722,8 @@ int vmoe_expert_backward(const void* saved, int64_t num_tokens, int32_t num_expe
  * grad_logits [T, E] bf16 nullable, else the auxiliary losses' logit
  * gradient for the device fp32 scalars grad_z / grad_lb / grad_cl
  * (nullable = 0; not all NULL unless weight_grad), plus with weight_grad the
- * routing weights' chain (vmoe_routing_weight_grad, its direct form and
- * vmoe_router_weight_bwd), the two added as bf16(a + b).
+ * routing weights' chain (the values of vmoe_routing_weight_grad, its direct
+ * form and vmoe_router_weight_bwd, in one launch), the two added as bf16(a + b).
  * ---------------------------------------------------------------------- */
 enum vmoe_moe_slot { VMOE_M_SELECTED = 0, VMOE_M_WEIGHTS, VMOE_M_LSE, VMOE_M_F_I32, VMOE_M_NSLOTS };
 int vmoe_moe_layout(int64_t num_tokens, int32_t num_experts, int32_t top_k, int32_t block_size,

@@ -19,6 +19,7 @@
 #include <mutex>
 
 #include "router_aux.h"
+#include "routing_wgrad.h"
 #include "vmoe_common.h"
 
 namespace vmoe {
@@ -213,8 +214,22 @@ extern "C" int vmoe_expert_forward(const void* selected, int32_t selected_is_int
 
 namespace vmoe {
 namespace {
-// vmoe_expert_backward; finish(gxg, rows, arow) turns the gathered dX rows into
-// grad_x on the main stream, beside the side stream's dW1.
+// What the GEMMs of the expert path's backward leave for the end of it: the
+// gathered dX rows (to be summed per token) and, where asked for, the dH GEMM's
+// row sums (the routing weights' gradients).
+struct ExpertGrads {
+  const uint16_t* gxg;
+  int64_t rows;
+  const int32_t* arow;
+  const float* row_dot;  // nullable; [rows][nblk]
+  int64_t nblk;
+  const float* row_weight;
+  DirectWgrad direct;
+};
+
+// vmoe_expert_backward up to that end, which is finish(ExpertGrads) on the main
+// stream, beside the side stream's dW1. zero_rest: blocks of row_dot at or past
+// an expert's width, which the dH GEMM does not write, are cleared.
 template <typename Finish>
 int expert_backward(
     const void* saved, int64_t num_tokens, int32_t num_experts, int32_t top_k,
@@ -222,7 +237,7 @@ int expert_backward(
     const uint16_t* w2, int64_t ldw2, const int32_t* ewo, const int32_t* widths, int64_t hidden,
     int64_t max_width, const uint16_t* grad_out, int64_t ldg, const uint16_t* grad_scale,
     uint16_t* grad_x, int64_t ldgx, uint16_t* grad_w1, int64_t ldgw1, uint16_t* grad_w2,
-    int64_t ldgw2, uint16_t* grad_weights, void* scratch, void* dw_workspace,
+    int64_t ldgw2, bool row_sums, bool zero_rest, void* scratch, void* dw_workspace,
     size_t dw_workspace_bytes, vmoe_stream_t stream, vmoe_stream_t side_stream,
     Finish&& finish) {
   Layout L;
@@ -242,14 +257,13 @@ int expert_backward(
   const uint16_t* pre = at<uint16_t>(saved, L.slot[VMOE_X_PRE]);
   uint16_t* ga = at<uint16_t>(scratch, L.b_ga);
   uint16_t* gxg = at<uint16_t>(scratch, L.b_gxg);
-  float* row_dot = grad_weights ? at<float>(scratch, L.b_rowdot) : nullptr;
+  float* row_dot = row_sums ? at<float>(scratch, L.b_rowdot) : nullptr;
   hipStream_t main_s = reinterpret_cast<hipStream_t>(stream);
   hipStream_t side_s = side_stream ? reinterpret_cast<hipStream_t>(side_stream) : main_s;
   const bool two = side_s != main_s;
   hipEvent_t* ev = nullptr;
   if (two) VMOE_TRY(events_for(&ev));
-  if (row_dot) {
-    // blocks at or past an expert's width are not written by the dH GEMM
+  if (row_dot && zero_rest) {
     const int64_t n = L.cap * L.nblk;
     VMOE_LAUNCH(zero_f32_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)),
                        dim3(256), 0, main_s, row_dot, n);
@@ -286,14 +300,9 @@ int expert_backward(
     if (st == VMOE_OK) st = st2;
   }
   VMOE_TRY(st);
-  if (grad_weights) {
-    VMOE_TRY(vmoe_routing_weight_grad(row_dot, L.nblk, (int32_t)L.nblk, L.cap, rw, arow, L.A,
-                                      grad_weights, stream));
-    VMOE_TRY(vmoe_routing_weight_grad_direct(grad_out, ldg, num_tokens, grad_scale, w2, ldw2,
-                                             pre, max_width, rw, arow, L.A, k, eto, ewo, widths,
-                                             E, hidden, L.cap, grad_weights, stream));
-  }
-  VMOE_TRY(finish(gxg, L.cap, arow));
+  VMOE_TRY(finish(ExpertGrads{gxg, L.cap, arow, row_dot, L.nblk, rw,
+                              DirectWgrad{grad_out, ldg, num_tokens, grad_scale, w2, ldw2, pre,
+                                          max_width, eto, ewo, widths, E, hidden}}));
   if (two) VMOE_TRY(order(main_s, side_s, ev[2]));
   return VMOE_OK;
 }
@@ -311,10 +320,20 @@ extern "C" int vmoe_expert_backward(
   return expert_backward(
       saved, num_tokens, num_experts, top_k, block_size, x, ldx, w1, ldw1, w2, ldw2, ewo, widths,
       hidden, max_width, grad_out, ldg, grad_scale, grad_x, ldgx, grad_w1, ldgw1, grad_w2, ldgw2,
-      grad_weights, scratch, dw_workspace, dw_workspace_bytes, stream, side_stream,
-      [&](const uint16_t* gxg, int64_t rows, const int32_t* arow) {
-        return vmoe_combine(gxg, rows, hidden, arow, nullptr, top_k, grad_x, ldgx, num_tokens,
-                            hidden, stream);
+      grad_weights != nullptr, true, scratch, dw_workspace, dw_workspace_bytes, stream,
+      side_stream, [&](const ExpertGrads& g) -> int {
+        if (grad_weights) {
+          const int64_t A = num_tokens * top_k;
+          const DirectWgrad& d = g.direct;
+          VMOE_TRY(vmoe_routing_weight_grad(g.row_dot, g.nblk, (int32_t)g.nblk, g.rows,
+                                            g.row_weight, g.arow, A, grad_weights, stream));
+          VMOE_TRY(vmoe_routing_weight_grad_direct(
+              grad_out, ldg, num_tokens, grad_scale, w2, ldw2, d.pre, max_width, g.row_weight,
+              g.arow, A, top_k, d.eto, ewo, widths, num_experts, hidden, g.rows, grad_weights,
+              stream));
+        }
+        return vmoe_combine(g.gxg, g.rows, hidden, g.arow, nullptr, top_k, grad_x, ldgx,
+                            num_tokens, hidden, stream);
       });
 }
 
@@ -325,8 +344,8 @@ extern "C" int vmoe_expert_backward(
 // logit gradient and, opt-in, the routing weights' chain into the logits.
 // saved = [expert saved block][selected int32 A][weights bf16 A][lse fp32 T]
 // [f_i fp32 E]; forward scratch = [expert forward scratch][partial rows]
-// [counted routing workspace][p_i fp32 E]; backward scratch = [expert
-// backward scratch][routing-weight gradient bf16 A][logit gradient bf16 T E].
+// [counted routing workspace][p_i fp32 E]; backward scratch = the expert
+// path's.
 // ---------------------------------------------------------------------------
 
 namespace vmoe {
@@ -340,7 +359,7 @@ struct MoeLayout {
   int64_t saved = 0;
   int64_t f_partial = 0, f_route_ws = 0, f_p_i = 0, f_scratch = 0;
   size_t route_ws_bytes = 0;
-  int64_t b_gw = 0, b_gl = 0, b_scratch = 0;
+  int64_t b_scratch = 0;
 };
 
 bool make_moe_layout(int64_t T, int E, int k, int b, int64_t hidden, int64_t max_w,
@@ -365,19 +384,8 @@ bool make_moe_layout(int64_t T, int E, int k, int b, int64_t hidden, int64_t max
   M.f_route_ws = M.f_partial + up256(4 * M.partial_rows * ((int64_t)E + 1));
   M.f_p_i = M.f_route_ws + up256((int64_t)M.route_ws_bytes);
   M.f_scratch = M.f_p_i + up256(4 * (int64_t)E);
-  M.b_gw = M.x.b_scratch;
-  M.b_gl = M.b_gw + up256(2 * A);
-  M.b_scratch = M.b_gl + up256(2 * T * (int64_t)E);
+  M.b_scratch = M.x.b_scratch;
   return true;
-}
-
-// a[i] = bf16(a[i] + b[i]) (fp32 sum, one rounding): two bf16 gradients of
-// one tensor added as autograd's accumulation adds them.
-__global__ void add_bf16_kernel(uint16_t* __restrict__ a, const uint16_t* __restrict__ b,
-                                int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    a[i] = (uint16_t)f32_to_bf16(bf16_to_f32(a[i]) + bf16_to_f32(b[i]));
 }
 
 }  // namespace
@@ -479,31 +487,24 @@ int moe_backward(
   if (!saved || !scratch) return VMOE_ERR_INVALID_ARG;
   const int E = num_experts;
   const int64_t T = num_tokens;
-  uint16_t* gw = weight_grad && grad_out && grad_logits ? at<uint16_t>(scratch, M.b_gw) : nullptr;
+  const bool chain = weight_grad && grad_out && grad_logits;  // through the routing weights
   const bool aux = grad_z || grad_lb || grad_cl;
   if (grad_logits) {
-    if (!aux && !gw) return VMOE_ERR_INVALID_ARG;  // the caller returns no logit gradient then
+    if (!aux && !chain) return VMOE_ERR_INVALID_ARG;  // the caller returns no logit gradient then
     if (!logits || !coef || !widths_normalized) return VMOE_ERR_INVALID_ARG;
   }
-  auto logit_grad = [&]() -> int {
-    const float* lse = at<float>(saved, M.slot[VMOE_M_LSE]);
-    const float* f_i32 = at<float>(saved, M.slot[VMOE_M_F_I32]);
-    if (aux)
-      VMOE_TRY(vmoe_router_aux_bwd(logits, E, T, E, lse, f_i32, coef, widths_normalized, grad_z,
-                                   grad_lb, grad_cl, grad_logits, E, stream));
-    if (gw) {
-      uint16_t* dst = aux ? at<uint16_t>(scratch, M.b_gl) : grad_logits;
-      VMOE_TRY(vmoe_router_weight_bwd(logits, E, T, E, top_k, normalize,
-                                      at<int32_t>(saved, M.slot[VMOE_M_SELECTED]), nullptr, gw,
-                                      top_k, dst, E, stream));
-      if (aux) {
-        const int64_t n = T * E;
-        VMOE_LAUNCH(add_bf16_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)),
-                    dim3(256), 0, reinterpret_cast<hipStream_t>(stream), grad_logits, dst, n);
-        VMOE_CHECK_LAUNCH();
-      }
-    }
-    return VMOE_OK;
+  const float* lse = at<float>(saved, M.slot[VMOE_M_LSE]);
+  const float* f_i32 = at<float>(saved, M.slot[VMOE_M_F_I32]);
+  auto aux_grad = [&] {
+    return vmoe_router_aux_bwd(logits, E, T, E, lse, f_i32, coef, widths_normalized, grad_z,
+                               grad_lb, grad_cl, grad_logits, E, stream);
+  };
+  auto chain_grad = [&](const ExpertGrads& g) {
+    return router_logit_grad(
+        LogitGrad{logits, T, E, top_k, normalize, at<int32_t>(saved, M.slot[VMOE_M_SELECTED]),
+                  lse, f_i32, coef, widths_normalized, grad_z, grad_lb, grad_cl, g.row_dot, g.nblk,
+                  (int)g.nblk, g.row_weight, g.arow, g.rows, g.direct, grad_logits},
+        stream);
   };
   // With the router's gradients in the same call, grad_x is formed where they
   // are: one launch reads the dX rows and writes grad_x once.
@@ -518,19 +519,20 @@ int moe_backward(
   if (grad_out) {
     VMOE_TRY(expert_backward(
         saved, T, E, top_k, block_size, x, ldx, w1, ldw1, w2, ldw2, ewo, widths, hidden, max_width,
-        grad_out, ldg, grad_scale, grad_x, ldgx, grad_w1, ldgw1, grad_w2, ldgw2, gw, scratch,
-        dw_workspace, dw_workspace_bytes, stream, side_stream,
-        [&](const uint16_t* gxg, int64_t rows, const int32_t* arow) -> int {
+        grad_out, ldg, grad_scale, grad_x, ldgx, grad_w1, ldgw1, grad_w2, ldgw2, chain, false,
+        scratch, dw_workspace, dw_workspace_bytes, stream, side_stream,
+        [&](const ExpertGrads& g) -> int {
+          if (chain) VMOE_TRY(chain_grad(g));
           if (!fused)
-            return vmoe_combine(gxg, rows, hidden, arow, nullptr, top_k, grad_x, ldgx, T, hidden,
-                                stream);
-          VMOE_TRY(logit_grad());
-          const RowSum sum = {gxg, hidden, rows, arow, top_k};
+            return vmoe_combine(g.gxg, g.rows, hidden, g.arow, nullptr, top_k, grad_x, ldgx, T,
+                                hidden, stream);
+          if (!chain) VMOE_TRY(aux_grad());
+          const RowSum sum = {g.gxg, hidden, g.rows, g.arow, top_k};
           return router_grad(&sum);
         }));
   }
   if (!grad_logits || fused) return VMOE_OK;
-  VMOE_TRY(logit_grad());
+  if (!chain) VMOE_TRY(aux_grad());
   return router ? router_grad(nullptr) : VMOE_OK;
 }
 }  // namespace

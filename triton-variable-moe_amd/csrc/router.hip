@@ -28,6 +28,7 @@
 #include <algorithm>
 
 #include "router_aux.h"
+#include "routing_wgrad.h"
 #include "vmoe_common.h"
 
 namespace vmoe {
@@ -649,6 +650,96 @@ __global__ __launch_bounds__(kRtThreads) void router_weight_bwd_kernel(
   }
 }
 
+// LogitGrad, one wave per token: lane j < k holds slot j for the weights'
+// gradient and their chain (as routing_wgrad_kernel and
+// router_weight_bwd_kernel), then lane l holds experts l, l + 64, .... The
+// launches it stands for (a fill of the row sums, the weights' gradient, its
+// direct form, the chain, the losses' gradient and an add) took 26 us and five
+// launch gaps of a 310 us step at 4101 tokens, 64 experts, k = 8; this one 7.
+template <int VPL>
+__global__ __launch_bounds__(kRtThreads) void router_logit_grad_kernel(LogitGrad a) {
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const bool aux = a.g_z || a.g_lb || a.g_cl;
+  const float invT = 1.0f / (float)a.T;
+  const float gz = a.g_z ? *a.g_z : 0.0f, glb = a.g_lb ? *a.g_lb : 0.0f,
+              gcl = a.g_cl ? *a.g_cl : 0.0f;
+  const int E = a.E, k = a.k;
+  float ce[VPL];
+#pragma unroll
+  for (int v = 0; v < VPL; ++v) {
+    const int e = lane + v * kWave;
+    ce[v] = aux && e < E ? (glb * a.coef[e] * a.f_i32[e] + gcl * a.wn[e]) * invT : 0.0f;
+  }
+  for (int64_t t = (int64_t)blockIdx.x * kRtWaves + wv; t < a.T;
+       t += (int64_t)gridDim.x * kRtWaves) {
+    int e = -1;
+    int32_t row = -1;
+    float p = 0.0f, g = 0.0f;
+    bool tiny = false;
+    if (lane < k) {
+      e = a.sel[t * k + lane];
+      row = a.assignment_row[t * k + lane];
+      if (row >= 0 && row < a.rows && e >= 0 && e < E) {
+        const float w = a.row_weight[row];
+        tiny = fabsf(w) < kTinyWeight;
+        if (!tiny) {
+          // blocks past the expert's width are not written and would add zeros
+          const int nb = min((a.direct.widths[e] + 63) >> 6, a.max_blocks);
+          const float* rd = a.row_dot + (int64_t)row * a.ld_rd;
+          float s = 0.0f;
+#pragma unroll 4
+          for (int b = 0; b < nb; ++b) s += rd[b];
+          g = s / w;
+        }
+      }
+      if (e >= 0 && e < E)
+        p = sigmoidf(bf16_to_f32(a.logits[t * E + e]));
+      else
+        e = -1;
+    }
+    uint64_t mask = ballot64(tiny);
+    while (mask) {
+      const int src = __builtin_ctzll(mask);
+      mask &= mask - 1;
+      const float s = direct_wgrad(a.direct, __shfl(row, src), t);
+      if (lane == src) g = s;
+    }
+    g = RtElt<false>::rnd(g);
+    if (e < 0) g = 0.0f;
+    float dp = g;
+    if (a.norm) {
+      const float S = wave_sum_f32(p) + 1e-20f;
+      const float gp = wave_sum_f32(g * p);
+      dp = (g - gp / S) / S;
+    }
+    const float dl = dp * p * (1.0f - p);
+    float val[VPL];
+#pragma unroll
+    for (int v = 0; v < VPL; ++v) val[v] = 0.0f;
+    for (int j = 0; j < k; ++j) {
+      const int ej = __shfl(e, j, kWave);
+      const float dj = __shfl(dl, j, kWave);
+#pragma unroll
+      for (int v = 0; v < VPL; ++v)
+        if (ej == lane + v * kWave) val[v] = dj;
+    }
+    const float l = aux ? a.lse[t] : 0.0f;
+    const float zt = gz * 2.0f * l * invT;
+#pragma unroll
+    for (int v = 0; v < VPL; ++v) {
+      const int ee = lane + v * kWave;
+      if (ee >= E) continue;
+      float d = RtElt<false>::rnd(val[v]);
+      if (aux) {
+        const float x = bf16_to_f32(a.logits[t * E + ee]);
+        const float q = sigmoidf(x);
+        d = RtElt<false>::rnd(zt * expf(x - l) + ce[v] * q * (1.0f - q)) + d;
+      }
+      a.grad[t * E + ee] = (uint16_t)f32_to_bf16(d);
+    }
+  }
+}
+
 inline int vpl_of(int E) {
   int v = 1;
   while (v * kWave < E) v <<= 1;
@@ -1177,3 +1268,30 @@ extern "C" int vmoe_router_logits(const uint16_t* x, int64_t ldx, int64_t num_to
   VMOE_CHECK_LAUNCH();
   return VMOE_OK;
 }
+
+namespace vmoe {
+int router_logit_grad(const LogitGrad& a, vmoe_stream_t stream) {
+  if (a.T <= 0 || a.E <= 0 || a.k <= 0 || a.k > kWave || !a.logits || !a.sel || !a.grad ||
+      !a.row_dot || !a.row_weight || !a.assignment_row)
+    return VMOE_ERR_INVALID_ARG;
+  if (a.E > kRtMaxExperts) return VMOE_ERR_UNSUPPORTED;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const dim3 grid((unsigned)std::min<int64_t>((a.T + kRtWaves - 1) / kRtWaves, 4096));
+  switch (vpl_of(a.E)) {
+#define VMOE_LG_CASE(V)                                                              \
+  case V:                                                                            \
+    VMOE_LAUNCH(router_logit_grad_kernel<V>, grid, dim3(kRtThreads), 0, s, a);       \
+    break;
+    VMOE_LG_CASE(1)
+    VMOE_LG_CASE(2)
+    VMOE_LG_CASE(4)
+    VMOE_LG_CASE(8)
+    VMOE_LG_CASE(16)
+    VMOE_LG_CASE(32)
+#undef VMOE_LG_CASE
+    default: return VMOE_ERR_UNSUPPORTED;
+  }
+  VMOE_CHECK_LAUNCH();
+  return VMOE_OK;
+}
+}  // namespace vmoe

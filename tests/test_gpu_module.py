@@ -896,3 +896,48 @@ def test_losses_in_routing_launch_same_bits(E, T, device):
         got.append([out, f_i, *aux.values()])
     for a, b in zip(*got):
         assert bits_equal(a, b)
+
+
+@pytest.mark.parametrize("d,sizes,k,T,b", [
+    (8, [(2, 8)], 1, 1, 8),                 # one token, K below one k-step
+    (136, [(3, 72), (5, 24)], 2, 9, 8),     # remainders in rows, columns and K
+    (264, [(4, 136)], 2, 2335, 8),          # 76 x 5 tiles of the down projection: taken
+    (264, [(4, 136)], 2, 2336, 8),          # 77 x 5: not
+    (384, [(6, 256), (3, 384)], 3, 33, 128),  # two row blocks; K of 2 and 3 stages
+    (640, [(70, 576)], 4, 50, 64),          # K of 5 stages, 70 experts
+    (768, [(4, 128)], 2, 61, 1),            # rows without padding
+    (256, [(4, 512)], 2, 130, 512),         # row blocks of padding alone
+])
+@pytest.mark.parametrize("skew", [False, True])
+def test_few_rows_same_bits(d, sizes, k, T, b, skew, device):
+    """Layers with few tokens per expert run their projections in 64 x 64
+    tiles with a deep stage; output and gradients have the bits of the
+    per-kernel path (the 128 x 256 tiles). With the skewed routing the first
+    experts get every token, several row blocks of one expert."""
+    from triton_moe.kernels import grouped_gemm as gg
+
+    torch.manual_seed(5)
+    cfg = TritonMoEConfig(n_embd=d, expert_sizes=sizes, num_active_experts=k, block_size=b)
+    m = TritonMoEMLP(cfg).to(device).to(torch.bfloat16)
+    if skew:
+        bias = torch.arange(sum(c for c, _ in sizes), 0, -1, device=device) * 100.0
+        m.router.register_forward_hook(lambda mod, i, o: o + bias.to(o.dtype))
+    x = torch.randn(T, 1, d, device=device).to(torch.bfloat16)
+    g = torch.randn(T, 1, d, device=device).to(torch.bfloat16)
+    results = []
+    for fused in (True, False):
+        gg.FUSED_EXPERT_PATH = fused
+        try:
+            with torch.no_grad():
+                alone = m(x)[0]
+            xi = x.clone().requires_grad_(True)
+            m.zero_grad(set_to_none=True)
+            out = m(xi)[0]
+            out.backward(g)
+            assert bits_equal(alone, out.detach())
+            results.append((alone, xi.grad.clone(), m.w1.grad.clone(), m.w2.grad.clone()))
+        finally:
+            gg.FUSED_EXPERT_PATH = True
+    assert results[0][0].float().abs().max() > 0
+    for u, v in zip(*results):
+        assert bits_equal(u, v)

@@ -21,8 +21,9 @@ REPO = HERE.parent
 CSRC = HERE / "csrc"
 OUT = HERE / "triton_moe" / "libvmoe.so"
 OBJ = HERE / "_build"
-SOURCES = ["route.hip", "permute.hip", "permute_f32.hip", "gemm.hip", "gemm_f32.hip", "router.hip", "router_bwd.hip",
-           "expert.hip", "expert_f32.hip", "capi.hip"]
+SOURCES = ["route.hip", "permute.hip", "permute_f32.hip", "gemm.hip", "gemm_few_rows.hip",
+           "gemm_f32.hip", "router.hip", "router_bwd.hip", "expert.hip", "expert_f32.hip",
+           "capi.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

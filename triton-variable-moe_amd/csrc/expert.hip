@@ -187,11 +187,19 @@ int expert_forward(const void* selected, int32_t selected_is_int64, const uint16
         at<void>(scratch, L.f_route_ws), L.route_ws_bytes, stream));
   }
   // H' = bf16(w * relu(x[map] W1_e)^2), PRE = relu(z); Y' = H' W2_e; combine
-  VMOE_TRY(vmoe_gemm_up_fwd(x, ldx, num_tokens, gmap, w1, ldw1, h, pre, max_width,
-                            VMOE_ACT_RELU_SQUARED, rw, eto, ewo, widths, ptpe, E, hidden,
-                            max_width, L.cap, stream));
-  VMOE_TRY(vmoe_gemm_down_fwd(h, max_width, w2, ldw2, y, hidden, eto, ewo, widths, ptpe, E,
-                              hidden, max_width, L.cap, stream));
+  if (few_rows_fits(L.A, E, max_width))
+    VMOE_TRY(few_rows_up(x, ldx, num_tokens, gmap, w1, ldw1, h, pre, max_width, rw, eto, ewo,
+                         widths, ptpe, E, hidden, max_width, L.A, block_size, stream));
+  else
+    VMOE_TRY(vmoe_gemm_up_fwd(x, ldx, num_tokens, gmap, w1, ldw1, h, pre, max_width,
+                              VMOE_ACT_RELU_SQUARED, rw, eto, ewo, widths, ptpe, E, hidden,
+                              max_width, L.cap, stream));
+  if (few_rows_fits(L.A, E, hidden))
+    VMOE_TRY(few_rows_down(h, max_width, gmap, w2, ldw2, y, hidden, eto, ewo, widths, ptpe, E,
+                           hidden, max_width, L.A, block_size, stream));
+  else
+    VMOE_TRY(vmoe_gemm_down_fwd(h, max_width, w2, ldw2, y, hidden, eto, ewo, widths, ptpe, E,
+                                hidden, max_width, L.cap, stream));
   return vmoe_combine(y, L.cap, hidden, arow, nullptr, k, out, ldo, num_tokens, hidden, stream);
 }
 }  // namespace
@@ -247,7 +255,7 @@ int expert_backward(
   if (!saved || !x || !w1 || !w2 || !ewo || !widths || !grad_out || !grad_x || !grad_w1 ||
       !grad_w2 || !scratch || !dw_workspace || ldg < 0 || ldgx < hidden)
     return VMOE_ERR_INVALID_ARG;
-  const int E = num_experts, k = top_k;
+  const int E = num_experts;
   const int32_t* gmap = at<int32_t>(saved, L.slot[VMOE_X_GATHER_MAP]);
   const int32_t* arow = at<int32_t>(saved, L.slot[VMOE_X_ASSIGNMENT_ROW]);
   const int32_t* eto = at<int32_t>(saved, L.slot[VMOE_X_EXPERT_OFFSETS]);

@@ -61,6 +61,25 @@ int gemm_f32_down_bwd_ga(const float* grad_y, int64_t ldgy, const float* w2, int
                          int64_t hidden, int64_t max_width, int64_t rows_bound,
                          vmoe_stream_t stream);
 
+// gemm_few_rows.hip: the bf16 layer's up (relu^2, PRE and H') and down
+// projection where the experts get few tokens, with the bits of
+// vmoe_gemm_up_fwd / vmoe_gemm_down_fwd (pad rows of Y left unwritten where a
+// whole 64-row block is padding). few_rows_fits: whether a projection of `cols`
+// columns takes them; operands they don't take give VMOE_ERR_UNSUPPORTED, as
+// they do there.
+constexpr int64_t kFewRowsItems = 384;
+bool few_rows_fits(int64_t assignments, int64_t E, int64_t cols);
+int few_rows_up(const uint16_t* x, int64_t ldx, int64_t x_rows, const int32_t* map,
+                const uint16_t* w1, int64_t ldw1, uint16_t* h, uint16_t* pre, int64_t ldh,
+                const float* row_scale, const int32_t* eto, const int32_t* ewo,
+                const int32_t* widths, const int32_t* tpe, int E, int64_t hidden,
+                int64_t max_width, int64_t assignments, int block_size, vmoe_stream_t stream);
+int few_rows_down(const uint16_t* h, int64_t ldh, const int32_t* map, const uint16_t* w2,
+                  int64_t ldw2, uint16_t* y, int64_t ldy, const int32_t* eto,
+                  const int32_t* ewo, const int32_t* widths, const int32_t* tpe, int E,
+                  int64_t hidden, int64_t max_width, int64_t assignments, int block_size,
+                  vmoe_stream_t stream);
+
 }  // namespace vmoe
 
 #define VMOE_LAUNCH(K, G, B, SH, S, ...)                                                   \

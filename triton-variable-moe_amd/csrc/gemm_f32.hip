@@ -341,12 +341,16 @@ __device__ __forceinline__ int64_t b_ld(const F32Args& p) { return F == F_UP_DW 
 // 79-90 without.)
 constexpr uint32_t kOob = 0x80000000u;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t f32_rsrc(const float* b) {
-  const uint64_t v = reinterpret_cast<uint64_t>(b);
+// A workgroup-uniform value in scalar registers.
+__device__ __forceinline__ int64_t uniform(int64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return __builtin_amdgcn_make_buffer_rsrc(
-      reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), 0, 0x7FFFFFFF, 0x00020000);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// b in scalar registers (uniform)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t f32_rsrc(const float* b) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(b), 0, 0x7FFFFFFF, 0x00020000);
 }
 
 // The 4 floats at byte offset off, of which the first n are in the operand.
@@ -373,25 +377,28 @@ struct VecOp {
   uint32_t off[kRuns];  // bytes from base (+ k0 * step) of the thread's runs
   int n[kRuns];         // KCONTIG: row inside; else elements of the run inside
   __device__ __forceinline__ void init(const float* corner, int64_t ld, int64_t extent) {
-    base = corner;
-    step = KCONTIG ? 1 : ld;
+    base = reinterpret_cast<const float*>(uniform(reinterpret_cast<int64_t>(corner)));
+    step = KCONTIG ? 1 : uniform(ld);
 #pragma unroll
     for (int i = 0; i < kRuns; ++i) {
       int k, x;
       run_at<KCONTIG>(i, k, x);
-      n[i] = (int)min<int64_t>(extent - x, 4);
+      n[i] = extent - x < 4 ? (int)(extent - x) : 4;
       off[i] = (uint32_t)((KCONTIG ? x * ld + k : k * ld + x) * 4);
     }
   }
+  // 32-bit tests on `left`, the stage's k still inside (int64_t min compiles to
+  // conversions and a minimum in double).
   template <bool WIDE>
   __device__ __forceinline__ void load(float4 (&r)[kRuns], int64_t k0, int64_t K) const {
     const auto rs = f32_rsrc(base + k0 * step);
+    const int left = K - k0 < kBK ? (int)(K - k0) : kBK;
 #pragma unroll
     for (int i = 0; i < kRuns; ++i) {
       int k, x;
       run_at<KCONTIG>(i, k, x);
-      const int left = (int)min<int64_t>(K - k0 - k, 4);
-      r[i] = f32_run<WIDE>(rs, off[i], KCONTIG ? (n[i] > 0 ? left : 0) : (left > 0 ? n[i] : 0));
+      const int in = min(left - k, 4);
+      r[i] = f32_run<WIDE>(rs, off[i], KCONTIG ? (n[i] > 0 ? in : 0) : (in > 0 ? n[i] : 0));
     }
   }
 };
@@ -427,9 +434,11 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_f32_kernel(F32Args p) {
   int e;
   int64_t local;
   for (int64_t j = blockIdx.x >> 3; find_tile<F>(p, j, e, local); j += gridDim.x >> 3) {
-    const F32Prob q = f32_prob<F>(p, e);
+    F32Prob q = f32_prob<F>(p, e);
+    q.M = uniform(q.M); q.N = uniform(q.N); q.K = uniform(q.K);
+    q.t0 = uniform(q.t0); q.w0 = uniform(q.w0); q.w = uniform(q.w);
     const int64_t tn_count = cdiv64(q.N, kT);
-    const int64_t m0 = (local / tn_count) * kT, n0 = (local % tn_count) * kT;
+    const int64_t m0 = uniform((local / tn_count) * kT), n0 = uniform((local % tn_count) * kT);
     f32x16_t acc, acc_up;
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[v] = acc_up[v] = 0.0f;

@@ -941,3 +941,35 @@ def test_few_rows_same_bits(d, sizes, k, T, b, skew, device):
     assert results[0][0].float().abs().max() > 0
     for u, v in zip(*results):
         assert bits_equal(u, v)
+
+
+@pytest.mark.parametrize("mode", ["router_in_node", "hooked_router", "weight_grad", "float32"])
+def test_checkpointed_step_same_bits(mode, device):
+    """The layer with its auxiliary losses under non-reentrant activation
+    checkpointing, which allows each saved tensor one unpacking per backward:
+    gradients and losses of the plain step, bit for bit."""
+    from torch.utils.checkpoint import checkpoint
+
+    dt = torch.float32 if mode == "float32" else torch.bfloat16
+    torch.manual_seed(2)
+    cfg = TritonMoEConfig(n_embd=128, expert_sizes=[(4, 128), (4, 64)], num_active_experts=2,
+                          routing_weight_grad=mode == "weight_grad")
+    m = TritonMoEMLP(cfg).to(device).to(dt)
+    if mode == "hooked_router":
+        m.router.register_forward_hook(lambda mod, inp, out: None)
+    x = torch.randn(2, 150, 128, device=device).to(dt)
+    g = torch.randn(2, 150, 128, device=device).to(dt)
+
+    def layer(t):
+        out, aux, _ = m(t)
+        return out, sum(v.float() for v in aux.values())
+
+    got = []
+    for run in (layer, lambda t: checkpoint(layer, t, use_reentrant=False)):
+        m.zero_grad(set_to_none=True)
+        xi = x.clone().requires_grad_(True)
+        out, aux = run(xi)
+        ((out * g).sum() + 10 * aux).backward()
+        got.append([out.detach(), aux.detach(), xi.grad, *(p.grad for p in m.parameters())])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)

@@ -1241,7 +1241,8 @@ def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts, rou
     """(grad_logits, grad_x, grad_w1, grad_w2, grad_wr), None where not formed.
     router: (whether x, whether the router weight needs a gradient) of a node
     that holds the router Linear (vmoe_moe_router_backward), else None."""
-    logits, x_flat, w1, w2, saved = ctx.saved_tensors[:5]
+    # read once: each access unpacks every tensor (checkpointing allows one)
+    logits, x_flat, w1, w2, saved, *rest = ctx.saved_tensors
     widths, ewo, coef, wn, k, b, max_width, _, weight_grad = ctx.consts
     T, E, d, norm = ctx.dims
     dev = logits.device
@@ -1281,7 +1282,7 @@ def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts, rou
     extra = ()
     if router is not None and want_logits:
         need_x, need_wr = router
-        wr = ctx.saved_tensors[5]
+        (wr,) = rest
         if need_x and grad_x is None:
             grad_x = torch.empty(T, d, dtype=torch.bfloat16, device=dev)
         n = 0

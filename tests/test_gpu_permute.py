@@ -265,6 +265,35 @@ def test_padded_scatter_weight_grad_opt_in(device):
         assert bits_equal(yd.grad, _ref_gather(G, maps, k, wts))
 
 
+def test_padded_scatter_weight_grad_unpacks_saved_tensors_once(device):
+    """Saved-tensor hooks (activation checkpointing, offloading) see each saved
+    tensor unpacked once per backward, and the gradients are the plain ones."""
+    T, d, E, k, b = 96, 64, 4, 2, 16
+    x, sel, wts, r, maps = _setup(T, d, E, k, b, device, seed=3)
+    dev = lambda a: torch.as_tensor(a).to(device)  # noqa: E731
+    args = [dev(r[n]) for n in ("indices", "bin_ids")]
+    bins, pb = dev(r["bins"]), dev(r["padded_bins"])
+    gen = torch.Generator().manual_seed(4)
+    y = torch.randn(int(r["padded_bins"][-1]), d, generator=gen).to(torch.bfloat16).to(device)
+    G = torch.randn(T, d, generator=gen).to(torch.bfloat16).to(device)
+    got, packed, unpacked = [], [], []
+    for hooks in (False, True):
+        yd = y.clone().requires_grad_(True)
+        wd = wts.reshape(-1).to(device).requires_grad_(True)
+        pack = lambda t: packed.append(t) or len(packed) - 1  # noqa: E731
+        unpack = lambda i: unpacked.append(i) or packed[i]  # noqa: E731
+        if hooks:
+            with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+                out = padded_scatter_autograd(yd, *args, wd, bins, pb, k, weight_grad=True)
+        else:
+            out = padded_scatter_autograd(yd, *args, wd, bins, pb, k, weight_grad=True)
+        out.backward(G)
+        got.append((yd.grad, wd.grad))
+    assert packed and sorted(unpacked) == list(range(len(packed)))
+    for a, c in zip(*got):
+        assert bits_equal(a, c)
+
+
 @pytest.mark.parametrize("T,d,E,k,b", [(128, 128, 4, 2, 128), (1024, 256, 8, 2, 128),
                                        (300, 100, 5, 2, 8), (257, 2058, 7, 3, 64)])
 def test_f32_gather_combine_and_weight_grad(T, d, E, k, b, device):

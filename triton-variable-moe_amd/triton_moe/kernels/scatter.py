@@ -73,13 +73,14 @@ class PaddedScatterOp(torch.autograd.Function):
     @custom_bwd(device_type="cuda")
     @once_differentiable
     def backward(ctx, grad_output):
-        rs, weights = ctx.saved_tensors[:2]
+        # read once: each access unpacks every tensor (checkpointing allows one)
+        rs, weights, *rest = ctx.saved_tensors
         grad_x = None
         if ctx.needs_input_grad[0]:
             grad_x = gather_rows(grad_output, rs, ctx.top_k, ctx.total_padded, weights=weights)
         grad_w = None
         if ctx.weight_grad and ctx.needs_input_grad[3]:
-            x, ar = ctx.saved_tensors[2:]
+            x, ar = rest
             grad_w = combine_weight_grad(grad_output, x, ar, ctx.top_k).to(weights.dtype)
             grad_w = grad_w.reshape(weights.shape)
         return grad_x, None, None, grad_w, None, None, None, None

@@ -973,3 +973,28 @@ def test_checkpointed_step_same_bits(mode, device):
         got.append([out.detach(), aux.detach(), xi.grad, *(p.grad for p in m.parameters())])
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_losses_accumulate_in_place(dtype, device):
+    """A training loop may sum the losses into the first of them in place; the
+    gradients are those of the plain sum."""
+    torch.manual_seed(4)
+    cfg = TritonMoEConfig(n_embd=64, expert_sizes=[(8, 64)], num_active_experts=2)
+    m = TritonMoEMLP(cfg).to(device).to(dtype)
+    x = torch.randn(1, 90, 64, device=device).to(dtype)
+    got = []
+    for in_place in (False, True):
+        m.zero_grad(set_to_none=True)
+        _, aux, _ = m(x)
+        loss = aux["router_z_loss"]
+        for key in ("load_balance_loss", "compute_loss"):
+            term = aux[key].to(dtype)
+            if in_place:
+                loss += term
+            else:
+                loss = loss + term
+        loss.backward()
+        got.append((loss.detach(), m.router.weight.grad.clone()))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)

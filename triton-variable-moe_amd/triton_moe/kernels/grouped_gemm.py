@@ -1347,13 +1347,15 @@ class MoELayerOpF32(torch.autograd.Function):
         saved = torch.empty(plan[0], dtype=torch.uint8, device=dev)
         scratch = torch.empty(plan[1], dtype=torch.uint8, device=dev)
         out = torch.empty(T, d, **f32)
-        losses = torch.empty(3, **f32)  # z, load balance, compute
+        # z in storage of its own, so that the others may be added to it in place
+        z = torch.empty((), **f32)
+        losses = torch.empty(2, **f32)  # load balance, compute
         f_i = torch.empty(E, **f32)
         st = plan[3](logits.data_ptr(), T, E, top_k, int(bool(normalize)), block_size,
                      x_flat.data_ptr(), x_flat.stride(0), w1.data_ptr(), w1.stride(0),
                      w2.data_ptr(), w2.stride(0), ewo.data_ptr(), widths.data_ptr(), d, max_width,
                      coef.data_ptr(), wn.data_ptr(), saved.data_ptr(), scratch.data_ptr(),
-                     out.data_ptr(), d, losses.data_ptr(), losses.data_ptr() + 4, f_i.data_ptr(),
+                     out.data_ptr(), d, z.data_ptr(), losses.data_ptr(), f_i.data_ptr(),
                      _lib.stream(dev))
         if st != _lib.OK:
             _lib.check(st, "vmoe_moe_f32_forward")
@@ -1361,7 +1363,7 @@ class MoELayerOpF32(torch.autograd.Function):
         ctx.consts = consts
         ctx.mark_non_differentiable(f_i)
         ctx.set_materialize_grads(False)  # as MoELayerOp
-        return out, losses[0], losses[1], losses[2], f_i
+        return out, z, losses[0], losses[1], f_i
 
     @staticmethod
     @once_differentiable

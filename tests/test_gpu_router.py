@@ -407,3 +407,13 @@ def test_router_linear_differentiable_twice(device):
     assert torch.allclose(jv.float(), lin(x).detach().float(), atol=1e-1)
     per = torch.func.vmap(torch.func.grad(lambda t: lin(t[None]).float().sum()))(x.detach())
     assert per.shape == x.shape
+
+
+def test_router_linear_compiles_whole(device):
+    """On the GPU too the router traces as one graph, the linear layer's."""
+    torch.manual_seed(0)
+    lin = RouterLinear(64, 16, bias=False).to(device).to(torch.bfloat16)
+    x = torch.randn(40, 64, device=device).to(torch.bfloat16).requires_grad_(True)
+    torch._dynamo.reset()
+    out = torch.compile(lin, fullgraph=True, backend="eager")(x)
+    assert torch.equal(out, F.linear(x, lin.weight))

@@ -180,3 +180,22 @@ def test_load_balance_coef_from_group_buffers(sizes):
         ref = (m.group_sizes.double() * (fp @ memb)).mean()
     # coef is fp32 (size / num_groups rounded once)
     assert (coef.double() * f * p).sum().item() == pytest.approx(ref.item(), rel=1e-6)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_router_linear_compiles_whole(dtype):
+    """The router traces as the plain linear layer it is, by torch.compile (one
+    graph, no break) and by torch.fx, with the linear layer's values and
+    gradients."""
+    from triton_moe.kernels.router import RouterLinear
+
+    torch.manual_seed(0)
+    lin = RouterLinear(16, 8, bias=False).to(dtype)
+    x = torch.randn(5, 16).to(dtype).requires_grad_(True)
+    torch._dynamo.reset()
+    out = torch.compile(lin, fullgraph=True, backend="eager")(x)
+    ref = torch.nn.functional.linear(x, lin.weight)
+    assert torch.equal(out, ref) and torch.equal(torch.fx.symbolic_trace(lin)(x), ref)
+    for a, b in zip(torch.autograd.grad(out.sum(), (x, lin.weight)),
+                    torch.autograd.grad(ref.sum(), (x, lin.weight))):
+        assert torch.equal(a, b)

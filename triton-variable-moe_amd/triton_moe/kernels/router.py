@@ -161,10 +161,11 @@ def router_bwd(g: torch.Tensor, x2d: torch.Tensor, wr: torch.Tensor, need_x: boo
 
 def _eager_call(*tensors: torch.Tensor) -> bool:
     """Plain tensors outside every transform that must see torch operators
-    (tracing, torch.func, forward-mode AD, dispatch modes)."""
-    return (all((type(t) is torch.Tensor or type(t) is nn.Parameter) and
+    (tracing, torch.func, forward-mode AD, dispatch modes). Compilation is
+    asked for first: the other tests are not traceable."""
+    return (not torch.compiler.is_compiling() and not torch.jit.is_tracing() and
+            all((type(t) is torch.Tensor or type(t) is nn.Parameter) and
                 torch._C._has_storage(t) for t in tensors) and
-            not torch.compiler.is_compiling() and not torch.jit.is_tracing() and
             torch._C._functorch.peek_interpreter_stack() is None and
             torch.autograd.forward_ad._current_level < 0 and
             torch._C._len_torch_dispatch_stack() == 0)

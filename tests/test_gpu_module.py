@@ -998,3 +998,36 @@ def test_losses_accumulate_in_place(dtype, device):
         got.append((loss.detach(), m.router.weight.grad.clone()))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("E", [8, 12])
+def test_router_only_training_keeps_routing_weight_gradient(E, device):
+    """With routing_weight_grad and everything but the router frozen, the
+    routing weights' chain still reaches the router, alone and beside the
+    losses' gradient: the per-kernel path's gradient."""
+    from triton_moe.kernels import grouped_gemm as gg
+
+    torch.manual_seed(6)
+    cfg = TritonMoEConfig(n_embd=64, expert_sizes=[(E, 64)], num_active_experts=2,
+                          routing_weight_grad=True)
+    m = TritonMoEMLP(cfg).to(device).to(torch.bfloat16)
+    m.w1.requires_grad_(False)
+    m.w2.requires_grad_(False)
+    x = torch.randn(1, 100, 64, device=device).to(torch.bfloat16)
+    g = torch.randn(1, 100, 64, device=device).to(torch.bfloat16)
+    for with_losses in (False, True):
+        got = []
+        for fused in (True, False):
+            gg.FUSED_EXPERT_PATH = fused
+            try:
+                m.router.weight.grad = None
+                out, aux, _ = m(x)
+                loss = (out * g).sum()
+                if with_losses:
+                    loss = loss + 10 * aux["load_balance_loss"]
+                loss.backward()
+                got.append(m.router.weight.grad)
+            finally:
+                gg.FUSED_EXPERT_PATH = True
+        assert got[0] is not None and got[0].abs().max() > 0
+        assert torch.equal(got[0], got[1])

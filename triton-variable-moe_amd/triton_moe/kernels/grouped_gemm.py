@@ -1249,7 +1249,8 @@ def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts, rou
     plan = _moe_plan(T, E, k, b, d, max_width, dev)
 
     gz, glb, gcl = _scalar_f32(g_z), _scalar_f32(g_lb), _scalar_f32(g_cl)
-    want_x = grad_out is not None and need_experts
+    # (the routing weights' gradients come out of the expert path's backward)
+    want_x = grad_out is not None and (need_experts or (weight_grad and need_logits))
     want_logits = need_logits and (
         gz is not None or glb is not None or gcl is not None or (weight_grad and want_x))
     grad_x = grad_w1 = grad_w2 = grad_logits = None

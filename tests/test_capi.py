@@ -222,6 +222,31 @@ def test_argument_checks_return_invalid_arg():
                                       None) == _lib.OK
 
 
+def test_router_backward_is_refused_before_any_launch():
+    """vmoe_moe_router_backward checks the router's operands and workspace
+    before it queues the layer's GEMMs: 256 tokens, 8 experts, width 64 (two
+    chunks of the weight gradient, 4 KiB of workspace), every pointer 16."""
+    lib = _lib.lib()
+    need = lib.vmoe_router_linear_bwd_workspace_bytes(256, 64, 8)
+    assert need == 2 * 8 * 64 * 4
+
+    def call(wr=16, ldwr=64, grad_wr=16, ldgwr=64, rws=16, rws_bytes=need, grad_x=16, k=2):
+        return lib.vmoe_moe_router_backward(
+            16, 16, 256, 8, k, 1, 64, 16, 64, 16, 512, 16, 64, 16, 16, 64, 64, 16, 16, 16, 64,
+            None, 16, 16, 16, 0, grad_x, 64, 16, 512, 16, 64, 16, 16, 16, 1 << 30, None, None,
+            wr, ldwr, grad_wr, ldgwr, 1, rws, rws_bytes)
+
+    for k in (2, 3):  # the rows are summed by the router's launch
+        assert call(k=k, rws_bytes=need - 1) == _lib.ERR_WORKSPACE
+        assert call(k=k, rws=None) == _lib.ERR_WORKSPACE
+        assert call(k=k, wr=8) == _lib.ERR_UNSUPPORTED
+        assert call(k=k, ldwr=60) == _lib.ERR_UNSUPPORTED
+        assert call(k=k, grad_wr=4) == _lib.ERR_UNSUPPORTED
+        assert call(k=k, ldgwr=56) == _lib.ERR_UNSUPPORTED
+        assert call(k=k, grad_x=8) == _lib.ERR_UNSUPPORTED
+        assert call(k=k, wr=None) == _lib.ERR_INVALID_ARG
+
+
 def test_check_maps_status_to_exceptions():
     with pytest.raises(ValueError):
         _lib.check(_lib.ERR_INVALID_ARG, "x")

@@ -271,48 +271,55 @@ int expert_backward(
   const bool two = side_s != main_s;
   hipEvent_t* ev = nullptr;
   if (two) VMOE_TRY(events_for(&ev));
-  if (row_dot && zero_rest) {
-    const int64_t n = L.cap * L.nblk;
-    VMOE_LAUNCH(zero_f32_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)),
-                       dim3(256), 0, main_s, row_dot, n);
-    VMOE_CHECK_LAUNCH();
-  }
-  // dW2 (needs only G and H') runs on the side stream beside dH; dW1 beside
-  // dX and the combine once GA exists. With one stream the two GEMMs of each
-  // pair share one launch, on half of the CUs each (gemm_pair_begin).
-  if (two) VMOE_TRY(order(side_s, main_s, ev[0]));
-  if (!two) gemm_pair_begin();
-  int st = vmoe_gemm_down_bwd_dh(grad_out, ldg, num_tokens, gmap, grad_scale, w2, ldw2, pre, rw,
-                                 ga, max_width, eto, ewo, widths, ptpe, E, hidden, max_width,
-                                 L.cap, row_dot, L.nblk, stream);
-  if (st == VMOE_OK)
-    st = vmoe_gemm_down_bwd_dw(h, max_width, grad_out, ldg, num_tokens, gmap, grad_scale, grad_w2,
-                               ldgw2, eto, ewo, widths, ptpe, E, hidden, max_width, L.cap,
-                               dw_workspace, dw_workspace_bytes,
-                               reinterpret_cast<vmoe_stream_t>(side_s));
-  if (!two) {
-    const int st2 = gemm_pair_end();
-    if (st == VMOE_OK) st = st2;
-  }
-  VMOE_TRY(st);
-  if (two) VMOE_TRY(order(side_s, main_s, ev[1]));
-  if (!two) gemm_pair_begin();
-  st = vmoe_gemm_up_bwd_dw(x, ldx, num_tokens, gmap, ga, max_width, grad_w1, ldgw1, eto, ewo,
-                           widths, ptpe, E, hidden, max_width, L.cap, dw_workspace,
-                           dw_workspace_bytes, reinterpret_cast<vmoe_stream_t>(side_s));
-  if (st == VMOE_OK)
-    st = vmoe_gemm_up_bwd_dx(ga, max_width, w1, ldw1, gxg, hidden, eto, ewo, widths, ptpe, E,
-                             hidden, max_width, L.cap, stream);
-  if (!two) {
-    const int st2 = gemm_pair_end();
-    if (st == VMOE_OK) st = st2;
-  }
-  VMOE_TRY(st);
-  VMOE_TRY(finish(ExpertGrads{gxg, L.cap, arow, row_dot, L.nblk, rw,
+  const int status = [&]() -> int {
+    if (row_dot && zero_rest) {
+      const int64_t n = L.cap * L.nblk;
+      VMOE_LAUNCH(zero_f32_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)),
+                         dim3(256), 0, main_s, row_dot, n);
+      VMOE_CHECK_LAUNCH();
+    }
+    // dW2 (needs only G and H') runs on the side stream beside dH; dW1 beside
+    // dX and the combine once GA exists. With one stream the two GEMMs of each
+    // pair share one launch, on half of the CUs each (gemm_pair_begin).
+    if (two) VMOE_TRY(order(side_s, main_s, ev[0]));
+    if (!two) gemm_pair_begin();
+    int st = vmoe_gemm_down_bwd_dh(grad_out, ldg, num_tokens, gmap, grad_scale, w2, ldw2, pre, rw,
+                                   ga, max_width, eto, ewo, widths, ptpe, E, hidden, max_width,
+                                   L.cap, row_dot, L.nblk, stream);
+    if (st == VMOE_OK)
+      st = vmoe_gemm_down_bwd_dw(h, max_width, grad_out, ldg, num_tokens, gmap, grad_scale, grad_w2,
+                                 ldgw2, eto, ewo, widths, ptpe, E, hidden, max_width, L.cap,
+                                 dw_workspace, dw_workspace_bytes,
+                                 reinterpret_cast<vmoe_stream_t>(side_s));
+    if (!two) {
+      const int st2 = gemm_pair_end();
+      if (st == VMOE_OK) st = st2;
+    }
+    VMOE_TRY(st);
+    if (two) VMOE_TRY(order(side_s, main_s, ev[1]));
+    if (!two) gemm_pair_begin();
+    st = vmoe_gemm_up_bwd_dw(x, ldx, num_tokens, gmap, ga, max_width, grad_w1, ldgw1, eto, ewo,
+                             widths, ptpe, E, hidden, max_width, L.cap, dw_workspace,
+                             dw_workspace_bytes, reinterpret_cast<vmoe_stream_t>(side_s));
+    if (st == VMOE_OK)
+      st = vmoe_gemm_up_bwd_dx(ga, max_width, w1, ldw1, gxg, hidden, eto, ewo, widths, ptpe, E,
+                               hidden, max_width, L.cap, stream);
+    if (!two) {
+      const int st2 = gemm_pair_end();
+      if (st == VMOE_OK) st = st2;
+    }
+    VMOE_TRY(st);
+    return finish(ExpertGrads{gxg, L.cap, arow, row_dot, L.nblk, rw,
                               DirectWgrad{grad_out, ldg, num_tokens, grad_scale, w2, ldw2, pre,
-                                          max_width, eto, ewo, widths, E, hidden}}));
-  if (two) VMOE_TRY(order(main_s, side_s, ev[2]));
-  return VMOE_OK;
+                                          max_width, eto, ewo, widths, E, hidden}});
+  }();
+  // The main stream waits for the side stream's GEMMs after a failed step too:
+  // the caller gives the buffers they use back in the main stream's order.
+  if (two) {
+    const int joined = order(main_s, side_s, ev[2]);
+    if (status == VMOE_OK) return joined;
+  }
+  return status;
 }
 }  // namespace
 }  // namespace vmoe
@@ -518,6 +525,13 @@ int moe_backward(
   // are: one launch reads the dX rows and writes grad_x once.
   const bool fused = router && router->need_x && grad_logits && grad_out &&
                      top_k <= kRowSumSlots && E <= kRowSumExperts;
+  const RowSum row_sum = {at<uint16_t>(scratch, M.x.b_gxg), hidden, M.x.cap,
+                          at<int32_t>(saved, M.x.slot[VMOE_X_ASSIGNMENT_ROW]), top_k};
+  if (router && grad_logits)  // refused before anything is queued
+    VMOE_TRY(router_linear_bwd_check(grad_logits, x, ldx, router->wr, router->ldwr, T, hidden, E,
+                                     router->need_x ? grad_x : nullptr, ldgx, router->grad_wr,
+                                     router->ldgwr, router->ws, router->ws_bytes,
+                                     fused ? &row_sum : nullptr));
   auto router_grad = [&](const RowSum* sum) {
     return router_linear_bwd(grad_logits, x, ldx, router->wr, router->ldwr, T, hidden, E,
                              router->need_x ? grad_x : nullptr, ldgx, grad_out != nullptr,
@@ -535,8 +549,7 @@ int moe_backward(
             return vmoe_combine(g.gxg, g.rows, hidden, g.arow, nullptr, top_k, grad_x, ldgx, T,
                                 hidden, stream);
           if (!chain) VMOE_TRY(aux_grad());
-          const RowSum sum = {g.gxg, hidden, g.rows, g.arow, top_k};
-          return router_grad(&sum);
+          return router_grad(&row_sum);
         }));
   }
   if (!grad_logits || fused) return VMOE_OK;

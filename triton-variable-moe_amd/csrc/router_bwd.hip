@@ -383,11 +383,14 @@ extern "C" size_t vmoe_router_linear_bwd_workspace_bytes(int64_t num_tokens, int
 }
 
 namespace vmoe {
-int router_linear_bwd(const uint16_t* grad_logits, const uint16_t* x, int64_t ldx,
-                      const uint16_t* weight, int64_t ldw, int64_t num_tokens, int64_t hidden,
-                      int32_t num_experts, uint16_t* grad_x, int64_t ldgx, int32_t accumulate,
-                      uint16_t* grad_weight, int64_t ldgw, void* workspace,
-                      size_t workspace_bytes, const RowSum* sum, vmoe_stream_t stream) {
+namespace {
+// The argument checks of router_linear_bwd and its kernel's operands; kmax: the
+// slots of the kernel instance that sums rows (0: none).
+int rb_args(const uint16_t* grad_logits, const uint16_t* x, int64_t ldx, const uint16_t* weight,
+            int64_t ldw, int64_t num_tokens, int64_t hidden, int32_t num_experts,
+            uint16_t* grad_x, int64_t ldgx, int32_t accumulate, uint16_t* grad_weight,
+            int64_t ldgw, void* workspace, size_t workspace_bytes, const RowSum* sum, RbArgs& p,
+            int& kmax) {
   if (num_tokens < 0 || hidden <= 0 || num_experts <= 0) return VMOE_ERR_INVALID_ARG;
   if (!grad_x && !grad_weight) return VMOE_OK;
   if (num_tokens == 0) return VMOE_ERR_INVALID_ARG;  // grad_weight would be left unwritten
@@ -396,23 +399,25 @@ int router_linear_bwd(const uint16_t* grad_logits, const uint16_t* x, int64_t ld
       hidden > INT32_MAX / 2 || num_tokens > INT32_MAX / 2 || !a16(grad_logits))
     return VMOE_ERR_UNSUPPORTED;
   // (ldx 0: one row for every token)
-  if (grad_weight && ((ldx != 0 && ldx < hidden) || ldx % 8 != 0 || !a16(x) || ldgw < hidden || ldgw % 4 != 0 ||
-                      (reinterpret_cast<uintptr_t>(grad_weight) & 7) != 0))
+  if (grad_weight &&
+      ((ldx != 0 && ldx < hidden) || ldx % 8 != 0 || !a16(x) || ldgw < hidden || ldgw % 4 != 0 ||
+       (reinterpret_cast<uintptr_t>(grad_weight) & 7) != 0))
     return VMOE_ERR_UNSUPPORTED;
   if (grad_x && (ldw < hidden || ldw % 8 != 0 || !a16(weight) || ldgx < hidden ||
                  ldgx % 8 != 0 || !a16(grad_x)))
     return VMOE_ERR_UNSUPPORTED;
-  RbArgs p{};
   p.g = grad_logits;
   p.x = x; p.ldx = ldx;
   p.w = weight; p.ldw = ldw;
   p.gx = grad_x; p.ldgx = ldgx; p.add = accumulate != 0;
   p.gw = grad_weight; p.ldgw = ldgw;
   p.T = num_tokens; p.E = num_experts; p.d = (int)hidden;
-  int kmax = 0;
+  kmax = 0;
   if (grad_x && sum) {
     if (!sum->y || !sum->arow || sum->k <= 0 || sum->ldy < hidden) return VMOE_ERR_INVALID_ARG;
-    if (sum->k > kRowSumSlots || num_experts > kRowSumExperts || sum->ldy % 8 != 0 || !a16(sum->y)) return VMOE_ERR_UNSUPPORTED;
+    if (sum->k > kRowSumSlots || num_experts > kRowSumExperts || sum->ldy % 8 != 0 ||
+        !a16(sum->y))
+      return VMOE_ERR_UNSUPPORTED;
     p.y = sum->y; p.ldy = sum->ldy; p.y_rows = sum->rows; p.arow = sum->arow; p.k = sum->k;
     kmax = sum->k <= 2 ? 2 : 8;
   }
@@ -423,6 +428,32 @@ int router_linear_bwd(const uint16_t* grad_logits, const uint16_t* x, int64_t ld
       return VMOE_ERR_WORKSPACE;
     p.partial = reinterpret_cast<float*>(workspace);
   }
+  return VMOE_OK;
+}
+}  // namespace
+
+int router_linear_bwd_check(const uint16_t* grad_logits, const uint16_t* x, int64_t ldx,
+                            const uint16_t* weight, int64_t ldw, int64_t num_tokens,
+                            int64_t hidden, int32_t num_experts, uint16_t* grad_x, int64_t ldgx,
+                            uint16_t* grad_weight, int64_t ldgw, void* workspace,
+                            size_t workspace_bytes, const RowSum* sum) {
+  RbArgs p{};
+  int kmax = 0;
+  return rb_args(grad_logits, x, ldx, weight, ldw, num_tokens, hidden, num_experts, grad_x, ldgx,
+                 0, grad_weight, ldgw, workspace, workspace_bytes, sum, p, kmax);
+}
+
+int router_linear_bwd(const uint16_t* grad_logits, const uint16_t* x, int64_t ldx,
+                      const uint16_t* weight, int64_t ldw, int64_t num_tokens, int64_t hidden,
+                      int32_t num_experts, uint16_t* grad_x, int64_t ldgx, int32_t accumulate,
+                      uint16_t* grad_weight, int64_t ldgw, void* workspace,
+                      size_t workspace_bytes, const RowSum* sum, vmoe_stream_t stream) {
+  RbArgs p{};
+  int kmax = 0;
+  const int st = rb_args(grad_logits, x, ldx, weight, ldw, num_tokens, hidden, num_experts, grad_x,
+                         ldgx, accumulate, grad_weight, ldgw, workspace, workspace_bytes, sum, p,
+                         kmax);
+  if (st != VMOE_OK || (!grad_x && !grad_weight)) return st;
   // up to 4 steps per workgroup while at least 4 workgroups per CU are left
   const int64_t steps = (num_tokens + kRbRows - 1) / kRbRows;
   p.iters = (int)std::max<int64_t>(1, std::min<int64_t>(4, steps * p.slabs / 1024));

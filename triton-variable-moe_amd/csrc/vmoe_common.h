@@ -51,6 +51,12 @@ int router_linear_bwd(const uint16_t* grad_logits, const uint16_t* x, int64_t ld
                       int32_t num_experts, uint16_t* grad_x, int64_t ldgx, int32_t accumulate,
                       uint16_t* grad_weight, int64_t ldgw, void* workspace,
                       size_t workspace_bytes, const RowSum* sum, vmoe_stream_t stream);
+// Its argument checks alone, for a caller that queues other work before it.
+int router_linear_bwd_check(const uint16_t* grad_logits, const uint16_t* x, int64_t ldx,
+                            const uint16_t* weight, int64_t ldw, int64_t num_tokens,
+                            int64_t hidden, int32_t num_experts, uint16_t* grad_x, int64_t ldgx,
+                            uint16_t* grad_weight, int64_t ldgw, void* workspace,
+                            size_t workspace_bytes, const RowSum* sum);
 
 // gemm_f32.hip: vmoe_gemm_f32_down_bwd_dh with the relu^2 rule in the epilogue,
 // ga = pre > 0 ? 2 gh pre : 0 for gh = grad_y W2_e^T (pre and ga share ldga):

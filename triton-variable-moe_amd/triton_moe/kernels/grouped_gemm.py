@@ -1167,8 +1167,43 @@ class MoELayerOp(torch.autograd.Function):
     the time."""
 
     @staticmethod
-    def forward(ctx, logits, x_flat, w1, w2, consts):
-        return _moe_forward(ctx, logits, x_flat, w1, w2, None, consts)
+    def forward(ctx, logits, x_flat, w1, w2, consts, wr=None):
+        widths, ewo, coef, wn, top_k, block_size, max_width, normalize, weight_grad = consts
+        T, d = x_flat.shape
+        E = widths.shape[0]
+        dev = x_flat.device
+        x_flat = _bf16(x_flat, "TritonMoEMLP x")
+        if not logits.is_contiguous() or logits.data_ptr() % 16:
+            logits = logits.clone(memory_format=torch.contiguous_format)
+        plan = _moe_plan(T, E, top_k, block_size, d, max_width, dev)
+        saved = torch.empty(plan[0], dtype=torch.uint8, device=dev)
+        scratch = torch.empty(plan[1], dtype=torch.uint8, device=dev)
+        out = torch.empty(T, d, dtype=torch.bfloat16, device=dev)
+        z = torch.empty((), dtype=torch.bfloat16, device=dev)
+        losses = torch.empty(2, dtype=torch.float32, device=dev)
+        f_i = torch.empty(E, dtype=torch.bfloat16, device=dev)
+        if T == 0:
+            z.zero_(), losses.zero_(), f_i.zero_()
+        st = plan[7](logits.data_ptr(), T, E, top_k, int(bool(normalize)), block_size,
+                     x_flat.data_ptr(), x_flat.stride(0), w1.data_ptr(), w1.stride(0),
+                     w2.data_ptr(), w2.stride(0), ewo.data_ptr(), widths.data_ptr(), d, max_width,
+                     coef.data_ptr(), wn.data_ptr(), saved.data_ptr(), scratch.data_ptr(),
+                     out.data_ptr(), d, z.data_ptr(), losses.data_ptr(), f_i.data_ptr(),
+                     _lib.stream(dev))
+        if st != _lib.OK:
+            _lib.check(st, "vmoe_moe_forward")
+        if wr is None:
+            ctx.save_for_backward(logits, x_flat, w1, w2, saved)
+        else:  # MoERouterLayerOp's
+            ctx.save_for_backward(logits, x_flat, w1, w2, saved, wr)
+        # the module's constant tables (buffers, never written in place)
+        ctx.consts = consts
+        ctx.dims = (T, E, d, int(bool(normalize)))
+        ctx.mark_non_differentiable(f_i)
+        # unused outputs arrive as None (not zeros), so a loss that leaves out
+        # the auxiliary losses gives the router no gradient, as in the reference
+        ctx.set_materialize_grads(False)
+        return out, z, losses[0], losses[1], f_i
 
     @staticmethod
     @once_differentiable
@@ -1189,7 +1224,7 @@ class MoERouterLayerOp(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x_flat, wr, w1, w2, consts):
-        return _moe_forward(ctx, F.linear(x_flat, wr), x_flat, w1, w2, wr, consts)
+        return MoELayerOp.forward(ctx, F.linear(x_flat, wr), x_flat, w1, w2, consts, wr)
 
     @staticmethod
     @once_differentiable
@@ -1199,42 +1234,6 @@ class MoERouterLayerOp(torch.autograd.Function):
             ctx, grad_out, g_z, g_lb, g_cl, need_x or need_wr, need_x or need_w1 or need_w2,
             (need_x, need_wr))
         return grad_x, grad_wr, grad_w1, grad_w2, None
-
-
-def _moe_forward(ctx, logits, x_flat, w1, w2, wr, consts):
-    widths, ewo, coef, wn, top_k, block_size, max_width, normalize, weight_grad = consts
-    T, d = x_flat.shape
-    E = widths.shape[0]
-    dev = x_flat.device
-    x_flat = _bf16(x_flat, "TritonMoEMLP x")
-    if not logits.is_contiguous() or logits.data_ptr() % 16:
-        logits = logits.clone(memory_format=torch.contiguous_format)
-    plan = _moe_plan(T, E, top_k, block_size, d, max_width, dev)
-    saved = torch.empty(plan[0], dtype=torch.uint8, device=dev)
-    scratch = torch.empty(plan[1], dtype=torch.uint8, device=dev)
-    out = torch.empty(T, d, dtype=torch.bfloat16, device=dev)
-    z = torch.empty((), dtype=torch.bfloat16, device=dev)
-    losses = torch.empty(2, dtype=torch.float32, device=dev)
-    f_i = torch.empty(E, dtype=torch.bfloat16, device=dev)
-    if T == 0:
-        z.zero_(), losses.zero_(), f_i.zero_()
-    st = plan[7](logits.data_ptr(), T, E, top_k, int(bool(normalize)), block_size,
-                 x_flat.data_ptr(), x_flat.stride(0), w1.data_ptr(), w1.stride(0),
-                 w2.data_ptr(), w2.stride(0), ewo.data_ptr(), widths.data_ptr(), d, max_width,
-                 coef.data_ptr(), wn.data_ptr(), saved.data_ptr(), scratch.data_ptr(),
-                 out.data_ptr(), d, z.data_ptr(), losses.data_ptr(), f_i.data_ptr(),
-                 _lib.stream(dev))
-    if st != _lib.OK:
-        _lib.check(st, "vmoe_moe_forward")
-    ctx.save_for_backward(logits, x_flat, w1, w2, saved, *(() if wr is None else (wr,)))
-    # the module's constant tables (buffers, never written in place)
-    ctx.consts = consts
-    ctx.dims = (T, E, d, int(bool(normalize)))
-    ctx.mark_non_differentiable(f_i)
-    # unused outputs arrive as None (not zeros), so a loss that leaves out
-    # the auxiliary losses gives the router no gradient, as in the reference
-    ctx.set_materialize_grads(False)
-    return out, z, losses[0], losses[1], f_i
 
 
 def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts, router):

@@ -190,7 +190,7 @@ class TritonMoEMLP(nn.Module):
 
     def _aux_tables(self, device):
         """fp32 load-balance coefficients and normalised widths on `device`."""
-        key = (str(device), self.expert_widths_normalized.dtype)
+        key = (device, self.expert_widths_normalized.dtype)
         cache = getattr(self, "_aux_cache", None)
         if cache is None or cache[0] != key:
             coef = self.load_balance_coef().to(device=device, dtype=torch.float32)
@@ -290,12 +290,13 @@ class TritonMoEMLP(nn.Module):
                                            r.row_src, r.assignment_row, w, k, self.config.n_embd)
         return output_flat, r.tokens_per_expert
 
-    def _layer_consts(self, coef, wn) -> tuple:
-        """MoELayerOp's constant tables and settings."""
+    def _layer_consts(self, device, grad: bool) -> tuple:
+        """MoELayerOp's constant tables and settings; grad: whether autograd
+        records the call."""
+        coef, wn = self._aux_tables(device)
         return (self.expert_widths_t, self.expert_weight_offsets_t, coef, wn,
                 self.num_active_experts, self.block_size, self.max_expert_width,
-                self.norm_topk_prob,
-                self.config.routing_weight_grad and torch.is_grad_enabled())
+                self.norm_topk_prob, grad and self.config.routing_weight_grad)
 
     def _router_in_node(self, x_flat) -> bool:
         """Whether the router Linear runs inside the layer's autograd node
@@ -320,11 +321,12 @@ class TritonMoEMLP(nn.Module):
         """x [batch, seq, n_embd] -> (output [batch, seq, n_embd], aux_loss dict, f_i)."""
         batch_size, seq_len, n_embd = x.shape
         x_flat = x.reshape(batch_size * seq_len, n_embd)  # rearrange "b s d -> (b s) d"
-        if torch.is_grad_enabled() and self._router_in_node(x_flat):
+        grad = torch.is_grad_enabled()
+        if grad and self._router_in_node(x_flat):
             # the router Linear too: its gradients come out of the same node
-            coef, wn = self._aux_tables(x_flat.device)
             out, z, lb, cl, f_i = MoERouterLayerOp.apply(
-                x_flat, self.router.weight, self.w1, self.w2, self._layer_consts(coef, wn))
+                x_flat, self.router.weight, self.w1, self.w2,
+                self._layer_consts(x_flat.device, grad))
             aux_loss = {"router_z_loss": z, "load_balance_loss": lb, "compute_loss": cl}
             return out.view(batch_size, seq_len, n_embd), aux_loss, f_i.to(x.dtype)
         router_logits = self.router(x_flat)
@@ -334,9 +336,9 @@ class TritonMoEMLP(nn.Module):
                                       not self._compact())) and
                 self.w1.dtype == torch.bfloat16 and router_logits.dtype == torch.bfloat16):
             # everything after the router Linear: one node, one call each way
-            coef, wn = self._aux_tables(router_logits.device)
             out, z, lb, cl, f_i = MoELayerOp.apply(
-                router_logits, x_flat, self.w1, self.w2, self._layer_consts(coef, wn))
+                router_logits, x_flat, self.w1, self.w2,
+                self._layer_consts(router_logits.device, grad))
             aux_loss = {"router_z_loss": z, "load_balance_loss": lb, "compute_loss": cl}
             return out.view(batch_size, seq_len, n_embd), aux_loss, f_i.to(x.dtype)
         if (x_flat.shape[0] > 0 and router_logits.is_cuda and self.num_experts <= 2048 and
@@ -344,16 +346,16 @@ class TritonMoEMLP(nn.Module):
                 self.w2.dtype == torch.float32 and x_flat.dtype == torch.float32 and
                 router_logits.dtype == torch.float32 and gg.FUSED_EXPERT_PATH and
                 _lib._launch_timer is None and
-                not (self.config.routing_weight_grad and torch.is_grad_enabled())):
-            coef, wn = self._aux_tables(router_logits.device)
+                not (grad and self.config.routing_weight_grad)):
             out, z, lb, cl, f_i = MoELayerOpF32.apply(
-                router_logits, x_flat, self.w1, self.w2, self._layer_consts(coef, wn))
+                router_logits, x_flat, self.w1, self.w2,
+                self._layer_consts(router_logits.device, grad))
             aux_loss = {"router_z_loss": z, "load_balance_loss": lb, "compute_loss": cl}
             return out.view(batch_size, seq_len, n_embd), aux_loss, f_i
         state = router_topk(router_logits, self.num_active_experts, self.norm_topk_prob,
                             route_hist=True)
         weights = state.weights
-        if self.config.routing_weight_grad and torch.is_grad_enabled():
+        if grad and self.config.routing_weight_grad:
             weights = RouterWeightOp.apply(router_logits, weights, state.selected,
                                            self.norm_topk_prob)
         output_flat, tokens_per_expert = self._experts(

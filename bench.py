@@ -572,8 +572,8 @@ def summary(name, r):
 def host_profile(name, device, steps):
     """Host side of the eager step of `name`: how fast the host issues steps
     (timed before the final synchronize) against how fast they complete, the
-    host time inside the two library calls of the layer (vmoe_moe_forward /
-    vmoe_moe_backward, bound ctypes functions timed around the call), and
+    host time inside the layer's library calls (the plan's bound ctypes
+    functions, timed around the call), and
     torch.profiler's CPU-only table over the same steps (self time per op, the
     autograd device thread included). Prints text, not a bench line."""
     import torch
@@ -611,8 +611,8 @@ def host_profile(name, device, steps):
 
     plans = dict(gg._MOE_PLANS)
     for key, plan in plans.items():
-        gg._MOE_PLANS[key] = plan[:7] + (timed(plan[7], "vmoe_moe_forward"),
-                                         timed(plan[8], "vmoe_moe_backward"))
+        gg._MOE_PLANS[key] = tuple(
+            timed(v, v.__name__) if callable(v) and not torch.is_tensor(v) else v for v in plan)
     try:
         for _ in range(steps):
             torch.cuda.synchronize()

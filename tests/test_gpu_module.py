@@ -1031,3 +1031,16 @@ def test_router_only_training_keeps_routing_weight_gradient(E, device):
                 gg.FUSED_EXPERT_PATH = True
         assert got[0] is not None and got[0].abs().max() > 0
         assert torch.equal(got[0], got[1])
+
+
+def test_bench_host_profile_runs(device, capsys):
+    """bench.py's host profile replaces the layer plan's functions by timed
+    ones; the step still runs and both calls it makes are reported."""
+    import bench
+    from triton_moe.kernels import grouped_gemm as gg
+
+    before = dict(gg._MOE_PLANS)
+    bench.host_profile("cfg1", device, 2)
+    text = capsys.readouterr().out
+    assert "vmoe_moe_forward: median" in text and "backward: median" in text
+    assert all(gg._MOE_PLANS[key] == plan for key, plan in before.items())

@@ -83,9 +83,9 @@ __global__ void zero_f32_kernel(float* __restrict__ p, int64_t n) {
 }
 
 // Events that order the backward's two streams, three per device (one per
-// hand-over), created on first use and kept for the process. An event is
-// recorded again only after the wait on its previous record was queued, so
-// reusing it loses no dependency.
+// hand-over), created on first use and kept for the process. Record and wait
+// are queued under one lock (order): an event that another thread records
+// again in between would leave the waiter without its dependency.
 constexpr int kMaxDevices = 64;
 std::mutex g_ev_mu;
 hipEvent_t g_ev[kMaxDevices][3];
@@ -106,6 +106,7 @@ int events_for(hipEvent_t** out) {
 }
 
 int order(hipStream_t waiter, hipStream_t signaler, hipEvent_t ev) {
+  std::lock_guard<std::mutex> g(g_ev_mu);
   if (hipEventRecord(ev, signaler) != hipSuccess ||
       hipStreamWaitEvent(waiter, ev, 0) != hipSuccess)
     return VMOE_ERR_LAUNCH;

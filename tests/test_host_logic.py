@@ -199,3 +199,19 @@ def test_router_linear_compiles_whole(dtype):
     for a, b in zip(torch.autograd.grad(out.sum(), (x, lin.weight)),
                     torch.autograd.grad(ref.sum(), (x, lin.weight))):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("name", ["_has_storage", "_len_torch_dispatch_stack"])
+def test_router_without_transform_probe(name, monkeypatch):
+    """A torch without one of the internals that tell an active transform keeps
+    the router on the linear layer's operators instead of failing."""
+    from triton_moe.kernels import router
+
+    assert router._transform_probe() is not None
+    x = torch.randn(3, 4)
+    assert router._eager_call(x)
+    monkeypatch.delattr(torch._C, name)
+    monkeypatch.setattr(router, "_in_transform", router._transform_probe())
+    assert router._in_transform is None and not router._eager_call(x)
+    lin = router.RouterLinear(4, 8, bias=False)
+    assert torch.equal(lin(x), nn.functional.linear(x, lin.weight))

@@ -159,16 +159,32 @@ def router_bwd(g: torch.Tensor, x2d: torch.Tensor, wr: torch.Tensor, need_x: boo
     return grad_x, grad_w
 
 
+def _transform_probe():
+    """Whether some transform other than plain autograd is active, as a
+    function; None where this torch lacks the means to tell (they are not
+    public API), and the router then stays on the linear layer's operators."""
+    try:
+        functorch_level = torch._C._functorch.peek_interpreter_stack
+        dispatch_modes = torch._C._len_torch_dispatch_stack
+        forward_ad = torch.autograd.forward_ad
+        torch._C._has_storage, forward_ad._current_level
+    except AttributeError:
+        return None
+    return lambda: (functorch_level() is not None or forward_ad._current_level >= 0 or
+                    dispatch_modes() > 0)
+
+
+_in_transform = _transform_probe()
+
+
 def _eager_call(*tensors: torch.Tensor) -> bool:
     """Plain tensors outside every transform that must see torch operators
     (tracing, torch.func, forward-mode AD, dispatch modes). Compilation is
     asked for first: the other tests are not traceable."""
     return (not torch.compiler.is_compiling() and not torch.jit.is_tracing() and
+            _in_transform is not None and
             all((type(t) is torch.Tensor or type(t) is nn.Parameter) and
-                torch._C._has_storage(t) for t in tensors) and
-            torch._C._functorch.peek_interpreter_stack() is None and
-            torch.autograd.forward_ad._current_level < 0 and
-            torch._C._len_torch_dispatch_stack() == 0)
+                torch._C._has_storage(t) for t in tensors) and not _in_transform())
 
 
 class RouterLinearOp(torch.autograd.Function):

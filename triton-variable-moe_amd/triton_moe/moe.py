@@ -25,7 +25,6 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from einops import rearrange
-from torch.nn.modules import module as nn_module
 
 from .kernels import (
     fused_route,
@@ -44,6 +43,11 @@ from .kernels.grouped_gemm import (CompactRoutedMoEOp, ExpertPathOp, GemmMeta, M
                                    f32_up_fwd, up_fwd)
 from .kernels.router import (RouterAuxOp, RouterLinear, RouterWeightOp, router_bwd_supported,
                              router_topk)
+
+
+# Whether hooks on every module's call are registered (not public API: without
+# it the router keeps its own call).
+_has_global_hook = getattr(nn.modules.module, "_has_any_global_hook", lambda: True)
 
 
 @dataclass
@@ -311,7 +315,7 @@ class TritonMoEMLP(nn.Module):
         return (gg.FUSED_EXPERT_PATH and _lib._launch_timer is None and not self._compact() and
                 r.bias is None and not r.use_logits_kernel and "forward" not in r.__dict__ and
                 not (r._forward_hooks or r._forward_pre_hooks or r._backward_hooks or
-                     r._backward_pre_hooks) and not nn_module._has_any_global_hook() and
+                     r._backward_pre_hooks) and not _has_global_hook() and
                 not torch.is_autocast_enabled() and router_bwd_supported(r.weight))
 
     @torch.compiler.disable

@@ -571,8 +571,8 @@ int vmoe_zero_tail_cols(uint16_t* buf, int64_t ld, const int32_t* eto, const int
  * fp32 grouped GEMMs: the float32 inputs of grouped_gemm_up / _down and their
  * backward and autograd functions (the reference's kernels are dtype-generic:
  * triton_moe/kernels/grouped_gemm.py:217-1162; its fp32 autograd tests:
- * tests/test_grouped_gemm_backward.py:151-208). fp32 in, fp32 fma
- * accumulation in k order, fp32 out. Metadata, rows_bound and the rows each
+ * tests/test_grouped_gemm_backward.py:151-208). fp32 in, fp32
+ * products and sums on the fp32 matrix instructions, fp32 out. Metadata, rows_bound and the rows each
  * expert covers are as for the bf16 GEMMs above; no alignment or multiple-of-8
  * requirement. Only the rows and columns the experts cover are written: the
  * caller zero-fills the rest (as the reference's torch.zeros outputs are).
@@ -748,6 +748,11 @@ int vmoe_moe_backward(const void* saved, const uint16_t* logits, int64_t num_tok
                       int64_t ldgw1, uint16_t* grad_w2, int64_t ldgw2, uint16_t* grad_logits,
                       void* scratch, void* dw_workspace, size_t dw_workspace_bytes,
                       vmoe_stream_t stream, vmoe_stream_t side_stream);
+
+/* 1 where the layer's up (cols = max_width) or down (cols = hidden) projection
+ * of num_assignments = num_tokens * top_k runs on 64 x 64 tiles (few tokens per
+ * expert), 0 where it runs on 128 x 256 ones; the results have the same bits. */
+int vmoe_moe_few_rows(int64_t num_assignments, int32_t num_experts, int64_t cols);
 
 /* vmoe_moe_backward and, where grad_logits is given, vmoe_router_linear_bwd on
  * it for logits = x wr^T: grad_wr (nullable) and, with need_x, the token

@@ -247,6 +247,71 @@ def test_router_backward_is_refused_before_any_launch():
         assert call(k=k, wr=None) == _lib.ERR_INVALID_ARG
 
 
+def test_router_linear_and_f32_layer_argument_checks():
+    """vmoe_router_linear_bwd and the float32 layer's calls refuse bad operands
+    before any launch (pointers are 16, sizes those of a 4 x 64 token layer)."""
+    lib = _lib.lib()
+    f = lib.vmoe_router_linear_bwd
+    ok = [16, 16, 64, 16, 64, 256, 64, 8, 16, 64, 0, 16, 64, 16, 1 << 20, None]
+
+    def bad(**kw):
+        names = ("g", "x", "ldx", "w", "ldw", "T", "d", "E", "gx", "ldgx", "acc", "gw", "ldgw",
+                 "ws", "n", "stream")
+        return f(*[kw.get(n, v) for n, v in zip(names, ok)])
+
+    assert bad(gx=None, gw=None) == _lib.OK  # nothing asked for
+    for kw in (dict(T=-1), dict(T=0), dict(d=0), dict(E=0), dict(g=None), dict(x=None),
+               dict(w=None)):
+        assert bad(**kw) == _lib.ERR_INVALID_ARG, kw
+    for kw in (dict(E=12), dict(E=136), dict(d=60), dict(g=8), dict(x=8), dict(ldx=56),
+               dict(ldx=68), dict(ldgw=60), dict(gw=4), dict(w=8), dict(ldw=56), dict(gx=8),
+               dict(ldgx=68)):
+        assert bad(**kw) == _lib.ERR_UNSUPPORTED, kw
+    for kw in (dict(ws=None), dict(ws=8), dict(n=16)):
+        assert bad(**kw) == _lib.ERR_WORKSPACE, kw
+    assert lib.vmoe_router_linear_bwd_workspace_bytes(0, 64, 8) == 0
+    assert lib.vmoe_router_linear_bwd_workspace_bytes(128, 64, 8) == 0  # one chunk
+
+    out = (ctypes.c_int64 * 3)()
+    assert lib.vmoe_moe_f32_layout(256, 4, 2, 128, 128, 256, out) == _lib.OK
+    cap = 256 * 2 + 4 * 127
+    assert out[0] >= 2 * 4 * cap * 256 and out[1] >= 4 * cap * 128
+    assert out[2] >= 4 * cap * (128 + 256) and all(v % 256 == 0 for v in out)
+    for args in ((-1, 4, 2, 128, 128, 256), (256, 0, 2, 128, 128, 256), (256, 4, 0, 128, 128, 256),
+                 (256, 4, 2, 0, 128, 256), (256, 128, 65, 128, 128, 256),
+                 (256, 2049, 2, 128, 128, 256)):
+        assert lib.vmoe_moe_f32_layout(*args, out) == _lib.ERR_INVALID_ARG, args
+    fwd = [16, 256, 4, 2, 1, 128, 16, 128, 16, 1024, 16, 128, 16, 16, 128, 256, 16, 16, 16, 16,
+           16, 128, 16, 16, 16, None]
+    assert lib.vmoe_moe_f32_forward(*[0 if i == 1 else v for i, v in enumerate(fwd)]) == _lib.OK
+    for i in (0, 6, 8, 10, 12, 13, 16, 17, 18, 19, 20, 22, 23, 24):  # every pointer
+        assert lib.vmoe_moe_f32_forward(
+            *[None if j == i else v for j, v in enumerate(fwd)]) == _lib.ERR_INVALID_ARG, i
+    bwd = [16, 16, 256, 4, 2, 128, 16, 128, 16, 1024, 16, 128, 16, 16, 128, 256, 16, 16, 16, 128,
+           16, 16, 16, 16, 128, 16, 1024, 16, 128, 16, 16, None]
+    assert lib.vmoe_moe_f32_backward(*[0 if i == 2 else v for i, v in enumerate(bwd)]) == _lib.OK
+    for i in (0, 6, 8, 10, 12, 13, 23, 25, 27, 30):
+        assert lib.vmoe_moe_f32_backward(
+            *[None if j == i else v for j, v in enumerate(bwd)]) == _lib.ERR_INVALID_ARG, i
+    # the losses' part alone: without a loss gradient, logits or their tables
+    aux = [None if i == 18 else v for i, v in enumerate(bwd)]
+    for drop in ((20, 21, 22), (1,), (16,), (17,)):
+        assert lib.vmoe_moe_f32_backward(
+            *[None if j in drop else v for j, v in enumerate(aux)]) == _lib.ERR_INVALID_ARG, drop
+
+
+def test_few_rows_rule():
+    """64 x 64 tiles up to 384 of them: row blocks with tokens (assignments / 64
+    and one more per expert that has any) times 64-column slabs."""
+    few = _lib.lib().vmoe_moe_few_rows
+    assert few(16, 8, 512) == 1 and few(16, 8, 768) == 1
+    assert few(4670, 4, 264) == 1 and few(4672, 4, 264) == 0  # 76 x 5 and 77 x 5
+    assert few(4672, 4, 256) == 1                             # 77 x 4
+    assert few(512, 64, 256) == 1 and few(512, 64, 1024) == 0
+    assert few(3, 128, 64 * 128) == 1 and few(4, 128, 64 * 128) == 0  # as many experts as rows
+    assert few(0, 8, 64) == 0 and few(16, 0, 64) == 0 and few(16, 8, 0) == 0
+
+
 def test_check_maps_status_to_exceptions():
     with pytest.raises(ValueError):
         _lib.check(_lib.ERR_INVALID_ARG, "x")

@@ -776,3 +776,34 @@ def test_cut_last_round_same_bits(activation, widths, device):
     whole, parts = up(0, E), [up(0, E // 2), up(E // 2, E)]
     for i in range(2):
         assert bits_equal(whole[i], torch.cat([p[i] for p in parts]))
+
+
+@pytest.mark.parametrize("form", ["down", "dX", "dH"])
+def test_cut_last_round_same_bits_other_forms(form, device):
+    """The same for the other row-tiled forms: 70 experts of 8 rows and 1000
+    result columns, 280 tiles, against two calls of 140."""
+    E, rows, N, K = 70, 8, 1000, 136
+    g = torch.Generator().manual_seed(13)
+
+    def normal(*shape, std=1.0):
+        return (torch.randn(*shape, generator=g) * std).to(torch.bfloat16).to(device)
+
+    hidden, w = (K, N) if form == "dH" else (N, K)
+    src = normal(E * rows, hidden if form == "dH" else w)
+    w1, w2 = normal(hidden, E * w, std=0.05), normal(E * w, hidden, std=0.05)
+    other = normal(E * rows, w if form == "dH" else hidden)
+
+    def run(e0, e1):
+        n, r = e1 - e0, slice(e0 * rows, e1 * rows)
+        i32 = dict(dtype=torch.int32, device=device)
+        eto = torch.arange(0, n * rows + 1, rows, **i32)
+        ewo = torch.arange(e0 * w, e1 * w + 1, w, **i32)
+        meta = (eto, ewo, torch.full((n,), w, **i32), torch.full((n,), rows, **i32))
+        if form == "down":
+            return grouped_gemm_down(src[r], w2, *meta, hidden)
+        if form == "dX":
+            return grouped_gemm_up_backward(src[r], other[r], w1, src[r], *meta, hidden,
+                                            "relu_squared")[0]
+        return grouped_gemm_down_backward(src[r], other[r], w2, *meta, hidden, w)[0]
+
+    assert bits_equal(run(0, E), torch.cat([run(0, E // 2), run(E // 2, E)]))

@@ -324,3 +324,39 @@ def test_f32_in_kernel_relu2_rule_matches_formed_ga(device):
     gx_b, gw_b = run(gh, _lib.ACT_RELU_SQUARED)
     assert torch.equal(gx_a, gx_b) and torch.equal(gw_a, gw_b)
     assert gx_a.abs().sum() > 0 and gw_a.abs().sum() > 0
+
+
+@pytest.mark.parametrize("gather", [False, True])
+def test_f32_operands_past_the_32_bit_offsets(gather, device):
+    """Operands whose rows lie 2^22 floats apart (16 MiB; offsets inside a tile,
+    and a gathered matrix as a whole, past 2^31 bytes) take the loads with
+    64-bit addresses: the bits of the same values in contiguous operands."""
+    rows, widths, d = [33, 0, 70], [36, 20, 65], 68
+    eto, tpe, offs = _meta(rows, widths, False)
+    xg, w1, w2 = (t.float() for t in _inputs(rows, widths, d, "relu_squared", 21))
+    g = torch.Generator().manual_seed(22)
+    P, W = sum(rows), sum(widths)
+    gy, gh = torch.randn(P, d, generator=g), torch.randn(P, max(widths), generator=g)
+    gm = torch.randint(-1, P, (P,), generator=g, dtype=torch.int32).to(device) if gather else None
+    meta = [_dev(v, device) for v in (eto, offs, widths, tpe)]
+    got = []
+    for far in (False, True):
+        def put(t):
+            t = t.to(device)
+            if not far:
+                return t
+            big = torch.empty(t.shape[0], 1 << 22, device=device)[:, :t.shape[1]]
+            assert big.stride(0) == 1 << 22
+            return big.copy_(t)
+
+        x, a, b, gy_, gh_ = put(xg), put(w1), put(w2), put(gy), put(gh)
+        h, pre = grouped_gemm_up(x, a, *meta, max(widths), "relu_squared", save_pre_act=True,
+                                 gather_map=gm)
+        h_, pre_ = put(h), put(pre)
+        got.append([h, pre, grouped_gemm_down(h_, b, *meta, d),
+                    *grouped_gemm_up_backward(gh_, x, a, pre_, *meta, d, "relu_squared",
+                                              gather_map=gm),
+                    *grouped_gemm_up_backward(gh_, x, a, pre_, *meta, d, "none", gather_map=gm),
+                    *grouped_gemm_down_backward(gy_, h_, b, *meta, d, max(widths))])
+    for near, far in zip(*got):
+        assert torch.equal(near, far)

@@ -842,7 +842,9 @@ def test_router_in_node_gradients(weight_grad, E, k, freeze, device):
     keeps its own linear node: outputs, losses and every gradient bit for bit
     (the input's is a rounded product, then a rounded sum, on both). With at
     most 64 experts and 8 slots the node's launch also sums the expert path's
-    rows; 72 experts or 9 slots leave that to the combine."""
+    rows; 72 experts or 9 slots leave that to the combine. Both form the
+    router's gradients with the same kernel, so a third run takes torch's own
+    linear backward: two bf16 roundings of fp32 sums in another order."""
     torch.manual_seed(3)
     cfg = TritonMoEConfig(n_embd=136, expert_sizes=[(4, 128), (E - 4, 64)],
                           num_active_experts=k, routing_weight_grad=weight_grad)
@@ -858,19 +860,26 @@ def test_router_in_node_gradients(weight_grad, E, k, freeze, device):
         for p in m.parameters():
             p.grad = None
         out, aux, f_i = m(xi)
-        names = {type(f[0]).__name__ for f in out.grad_fn.next_functions if f[0] is not None}
+        name = type(out.grad_fn.next_functions[0][0]).__name__  # below the output's view
         loss = (out * g).sum() + 10 * aux["router_z_loss"] + 10 * aux["load_balance_loss"]
         loss.backward()
-        return (names, out.detach(), aux["router_z_loss"].detach(), f_i, m.w1.grad, m.w2.grad,
+        return (name, out.detach(), aux["router_z_loss"].detach(), f_i, m.w1.grad, m.w2.grad,
                 xi.grad, m.router.weight.grad)
 
     a = step()
     h = m.router.register_forward_hook(lambda mod, inp, out: None)
     b = step()
     h.remove()
-    assert a[0] != b[0] or freeze in ("router", "x")  # the hooked router has a node of its own
+    assert (a[0], b[0]) == ("MoERouterLayerOpBackward", "MoELayerOpBackward")
     for u, v in zip(a[1:], b[1:]):
         assert (u is None) == (v is None) and (u is None or torch.equal(u, v))
+    m.router.forward = lambda t: torch.nn.functional.linear(t, m.router.weight)
+    c = step()
+    assert c[0] == "MoELayerOpBackward"
+    for u, v, what in ((a[6], c[6], "x"), (a[7], c[7], "router")):
+        assert (u is None) == (v is None)
+        if u is not None:
+            assert_close_norm(u, v, TIGHT, what)
 
 
 @pytest.mark.parametrize("E,T", [(72, 40), (128, 1531), (64, 300), (136, 200)])
@@ -898,24 +907,31 @@ def test_losses_in_routing_launch_same_bits(E, T, device):
         assert bits_equal(a, b)
 
 
-@pytest.mark.parametrize("d,sizes,k,T,b", [
-    (8, [(2, 8)], 1, 1, 8),                 # one token, K below one k-step
-    (136, [(3, 72), (5, 24)], 2, 9, 8),     # remainders in rows, columns and K
-    (264, [(4, 136)], 2, 2335, 8),          # 76 x 5 tiles of the down projection: taken
-    (264, [(4, 136)], 2, 2336, 8),          # 77 x 5: not
-    (384, [(6, 256), (3, 384)], 3, 33, 128),  # two row blocks; K of 2 and 3 stages
-    (640, [(70, 576)], 4, 50, 64),          # K of 5 stages, 70 experts
-    (768, [(4, 128)], 2, 61, 1),            # rows without padding
-    (256, [(4, 512)], 2, 130, 512),         # row blocks of padding alone
+@pytest.mark.parametrize("d,sizes,k,T,b,taken", [
+    (8, [(2, 8)], 1, 1, 8, (1, 1)),              # one token, K below one k-step
+    (136, [(3, 72), (5, 24)], 2, 9, 8, (1, 1)),  # remainders in rows, columns and K
+    (264, [(4, 136)], 2, 2335, 8, (1, 1)),       # 76 x 5 tiles of the down projection
+    (264, [(4, 136)], 2, 2336, 8, (1, 0)),       # 77 x 5
+    (384, [(6, 256), (3, 384)], 3, 33, 128, (1, 1)),  # two row blocks; K of 2 and 3 stages
+    (640, [(70, 576)], 4, 50, 64, (0, 0)),       # 73 x 9 and 73 x 10
+    (640, [(30, 576)], 4, 50, 64, (1, 1)),       # K of 5 stages
+    (768, [(4, 128)], 2, 61, 1, (1, 1)),         # rows without padding
+    (256, [(4, 512)], 2, 130, 512, (1, 1)),      # row blocks of padding alone
+    (64, [(70, 64)], 4, 50, 64, (1, 1)),         # more experts than lanes
 ])
 @pytest.mark.parametrize("skew", [False, True])
-def test_few_rows_same_bits(d, sizes, k, T, b, skew, device):
+def test_few_rows_same_bits(d, sizes, k, T, b, taken, skew, device):
     """Layers with few tokens per expert run their projections in 64 x 64
-    tiles with a deep stage; output and gradients have the bits of the
-    per-kernel path (the 128 x 256 tiles). With the skewed routing the first
-    experts get every token, several row blocks of one expert."""
+    tiles with a deep stage (taken: whether the up and the down projection do);
+    output and gradients have the bits of the per-kernel path (the 128 x 256
+    tiles). With the skewed routing the first experts get every token, several
+    row blocks of one expert."""
+    from triton_moe import _lib
     from triton_moe.kernels import grouped_gemm as gg
 
+    E = sum(c for c, _ in sizes)
+    few = _lib.lib().vmoe_moe_few_rows
+    assert (few(T * k, E, max(w for _, w in sizes)), few(T * k, E, d)) == taken
     torch.manual_seed(5)
     cfg = TritonMoEConfig(n_embd=d, expert_sizes=sizes, num_active_experts=k, block_size=b)
     m = TritonMoEMLP(cfg).to(device).to(torch.bfloat16)
@@ -1044,3 +1060,43 @@ def test_bench_host_profile_runs(device, capsys):
     text = capsys.readouterr().out
     assert "vmoe_moe_forward: median" in text and "backward: median" in text
     assert all(gg._MOE_PLANS[key] == plan for key, plan in before.items())
+
+
+@pytest.mark.parametrize("d,width,cut", [(136, 1000, "dH"), (1000, 136, "dX")])
+def test_cut_last_round_in_paired_backward_same_bits(d, width, cut, device):
+    """36 experts of 8 rows and 1000 columns give dH (or dX) 144 tiles: one
+    round and a cut second one on the half of the CUs that a paired launch has
+    (128 workgroups), less than a round on a launch of their own (256). The
+    gradients that come from them, the input's and (through the row sums of dH)
+    the router's, have the same bits; the expert weights' split sums differ in
+    their order."""
+    from triton_moe.kernels import grouped_gemm as gg
+
+    E, T, k = 36, 144, 2
+    torch.manual_seed(12)
+    cfg = TritonMoEConfig(n_embd=d, expert_sizes=[(E, width)], num_active_experts=k,
+                          block_size=8, routing_weight_grad=True)
+    m = TritonMoEMLP(cfg).to(device).to(torch.bfloat16)
+    bias = torch.zeros(T, E)  # every expert gets 8 tokens
+    t = torch.arange(T)
+    bias[t, t % E], bias[t, (t + 7) % E] = 3.0, 2.5
+    bias = bias.to(device).to(torch.bfloat16)
+    m.router.register_forward_hook(lambda mod, i, o: o * 0.125 + bias)
+    x = torch.randn(1, T, d, device=device).to(torch.bfloat16)
+    g = torch.randn(1, T, d, device=device).to(torch.bfloat16)
+    got = []
+    for side in (False, True):
+        gg.BACKWARD_SIDE_STREAM = side
+        try:
+            xi = x.clone().requires_grad_(True)
+            m.zero_grad(set_to_none=True)
+            out, _, f_i = m(xi)
+            out.backward(g)
+            got.append((xi.grad, m.router.weight.grad, m.w1.grad, m.w2.grad))
+        finally:
+            gg.BACKWARD_SIDE_STREAM = None
+    assert bool((f_i.float() * T * k).round().eq(8).all())
+    for a, b in zip(got[0][:2], got[1][:2]):
+        assert bits_equal(a, b)
+    for a, b in zip(got[0][2:], got[1][2:]):
+        assert_close_norm(a, b, TIGHT, cut)

@@ -218,6 +218,8 @@ def test_f32_one_call_path_same_bits_as_per_kernel_path(name, grad, device):
             m = _model(d, sizes, k, b, device)
             x = x0.clone().requires_grad_(True)
             out, aux, f_i = m(x)
+            node = type(out.grad_fn.next_functions[0][0]).__name__  # below the output's view
+            assert node == ("MoELayerOpF32Backward" if fused else "RoutedMoEOpF32Backward")
             losses = aux["router_z_loss"] + aux["load_balance_loss"] + aux["compute_loss"]
             if grad == "aux_only":
                 losses.backward()

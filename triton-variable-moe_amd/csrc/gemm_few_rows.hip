@@ -325,3 +325,9 @@ int few_rows_down(const uint16_t* h, int64_t ldh, const int32_t* map, const uint
 }
 
 }  // namespace vmoe
+
+extern "C" int vmoe_moe_few_rows(int64_t num_assignments, int32_t num_experts, int64_t cols) {
+  return num_assignments > 0 && num_experts > 0 &&
+                 vmoe::few_rows_fits(num_assignments, num_experts, cols)
+             ? 1 : 0;
+}

@@ -49,6 +49,7 @@ _SIGNATURES = {
                           _i64, _vp, _vp, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp,
                           _i32, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, ctypes.c_size_t,
                           _vp, _vp],
+    "vmoe_moe_few_rows": [_i64, _i32, _i64],
     "vmoe_moe_router_backward": [_vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, _i64, _vp, _i64,
                                  _vp, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp,
                                  _vp, _vp, _i32, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp,

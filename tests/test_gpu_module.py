@@ -1060,43 +1060,3 @@ def test_bench_host_profile_runs(device, capsys):
     text = capsys.readouterr().out
     assert "vmoe_moe_forward: median" in text and "backward: median" in text
     assert all(gg._MOE_PLANS[key] == plan for key, plan in before.items())
-
-
-@pytest.mark.parametrize("d,width,cut", [(136, 1000, "dH"), (1000, 136, "dX")])
-def test_cut_last_round_in_paired_backward_same_bits(d, width, cut, device):
-    """36 experts of 8 rows and 1000 columns give dH (or dX) 144 tiles: one
-    round and a cut second one on the half of the CUs that a paired launch has
-    (128 workgroups), less than a round on a launch of their own (256). The
-    gradients that come from them, the input's and (through the row sums of dH)
-    the router's, have the same bits; the expert weights' split sums differ in
-    their order."""
-    from triton_moe.kernels import grouped_gemm as gg
-
-    E, T, k = 36, 144, 2
-    torch.manual_seed(12)
-    cfg = TritonMoEConfig(n_embd=d, expert_sizes=[(E, width)], num_active_experts=k,
-                          block_size=8, routing_weight_grad=True)
-    m = TritonMoEMLP(cfg).to(device).to(torch.bfloat16)
-    bias = torch.zeros(T, E)  # every expert gets 8 tokens
-    t = torch.arange(T)
-    bias[t, t % E], bias[t, (t + 7) % E] = 3.0, 2.5
-    bias = bias.to(device).to(torch.bfloat16)
-    m.router.register_forward_hook(lambda mod, i, o: o * 0.125 + bias)
-    x = torch.randn(1, T, d, device=device).to(torch.bfloat16)
-    g = torch.randn(1, T, d, device=device).to(torch.bfloat16)
-    got = []
-    for side in (False, True):
-        gg.BACKWARD_SIDE_STREAM = side
-        try:
-            xi = x.clone().requires_grad_(True)
-            m.zero_grad(set_to_none=True)
-            out, _, f_i = m(xi)
-            out.backward(g)
-            got.append((xi.grad, m.router.weight.grad, m.w1.grad, m.w2.grad))
-        finally:
-            gg.BACKWARD_SIDE_STREAM = None
-    assert bool((f_i.float() * T * k).round().eq(8).all())
-    for a, b in zip(got[0][:2], got[1][:2]):
-        assert bits_equal(a, b)
-    for a, b in zip(got[0][2:], got[1][2:]):
-        assert_close_norm(a, b, TIGHT, cut)

@@ -431,28 +431,37 @@ struct Meta {
 // (equal shares of the k-steps, see build_meta), and its slot s works on
 // tile L * group + s of each. lin = L * l + s names the workgroup's split-K
 // partial slots.
+template <bool CUT>
 struct Range {
   int beg, end, stride, lin, slot;
-  // Round-robin: where an XCD's tiles are one round and up to a quarter of
-  // another, the tiles of that second round are cut along n into cut = 4
-  // pieces, so that four times as many workgroups share it; this workgroup
-  // takes piece `piece` of tile `tail` (-1: none). cut is 1 otherwise. A piece
-  // takes as many k-steps and staging instructions as its tile and a quarter
-  // of the bytes of B, so it pays where the GEMM streams weights (few rows per
-  // expert: 1531 tokens through 128 experts of 256-1024, up projection 104 ->
-  // 89 us); a step bound by staging (8192 tokens through 8 experts of 512)
-  // takes the same time with and without. After more rounds, or for a fuller
-  // last one (halves), it cost up to 1 %; with no full round before it (64
-  // tokens, 64 experts of 256) 20.3 -> 22.0 us.
-  int tail, piece, cut;
+  // CUT (the up projection): where an XCD's tiles are one round and up to a
+  // quarter of another, the tiles of that second round are cut along n into
+  // four pieces, so that four times as many workgroups share it; this workgroup
+  // takes piece `piece` of tile `tail` (-1: none). A piece takes as many
+  // k-steps and staging instructions as its tile and a quarter of the bytes of
+  // B, so it pays where the tail waits for weights: K at least kCutK, and few
+  // rows per expert (kCutRows). Forwards of 60 layers drawn with 260-310 tiles
+  // and 20-105 rows an expert, without / with the cut: 1.00-1.05 (mean 1.02)
+  // at K = 2048-4096, 0.99-1.04 at 1536, 0.98-1.02 at 1024; with 150-500 rows
+  // an expert at K = 1536-2048 0.97-1.01. 1531 tokens through 128 experts of
+  // 256-1024, K = 2048: the up projection 104 -> 89 us, the layer 226 -> 214.
+  // Not taken: more rounds, or a fuller last one in halves (up to 1 % slower),
+  // and no full round before it (64 tokens, 64 experts of 256: 20.3 -> 22.0
+  // us). The other forms gained nothing (the code spilled scalars in dH).
+  int tail, piece;
   // The workgroup's items in order: beg, beg + stride, ... below end, then the
   // tail; -1 past the last.
-  __device__ __forceinline__ int first() const { return beg < end ? beg : tail; }
+  __device__ __forceinline__ int last() const { return CUT ? tail : -1; }
+  __device__ __forceinline__ int first() const { return beg < end ? beg : last(); }
   __device__ __forceinline__ int next(int item) const {
-    return item >= end ? -1 : item + stride < end ? item + stride : tail;
+    return item + stride < end ? item + stride : item < end ? last() : -1;
   }
-  __device__ __forceinline__ int cut_of(int item) const { return item < end ? 1 : cut; }
+  // the piece of an item that the workgroup takes, -1: all of it
+  __device__ __forceinline__ int piece_of(int item) const {
+    return CUT && item >= end ? piece : -1;
+  }
 };
+constexpr int kCutK = 1536, kCutRows = 160;  // kCutRows: padded rows per expert
 
 // The workgroup's index among the p.grid workgroups of its GEMM. A paired
 // launch (grouped_gemm_pair_kernel) deals consecutive groups of 8 workgroups
@@ -464,13 +473,15 @@ __device__ __forceinline__ int vblock(const Args& p) {
   return p.paired ? ((b >> 4) << 3) | (b & 7) : b;
 }
 
-template <bool CONTIG>
-__device__ __forceinline__ Range item_range(const Args& p, int total, const int* lane_beg) {
+template <bool CONTIG, bool CUT>
+__device__ __forceinline__ Range<CUT> item_range(const Args& p, int total, const int* lane_beg) {
   const int G = p.grid, b = vblock(p);
   const int xcd = b & 7, per = G >> 3, j = b >> 3;
-  Range r;
+  Range<CUT> r;
   r.lin = xcd * per + j;
   r.slot = 0;
+  r.tail = -1;
+  r.piece = 0;
   if (CONTIG) {
     const int NL = G >> p.lsh;
     const int lane = xcd * (NL >> 3) + (j >> p.lsh);
@@ -479,19 +490,19 @@ __device__ __forceinline__ Range item_range(const Args& p, int total, const int*
     r.beg = lane_beg[lane];
     r.end = lane_beg[lane + 1];
     r.stride = 1;
-    r.tail = -1;
-    r.piece = 0;
-    r.cut = 1;
   } else {
-    const int first = __builtin_amdgcn_readfirstlane(lane_beg[xcd]);
-    const int count = __builtin_amdgcn_readfirstlane(lane_beg[xcd + 1]) - first;
-    const int rounds = udiv_small(count, per), rem = count - rounds * per;
-    r.cut = rounds == 1 && 4 * rem <= per ? 4 : 1;
-    r.beg = first + j;
-    r.end = r.cut > 1 ? first + rounds * per : first + count;
+    r.beg = lane_beg[xcd] + j;
+    r.end = lane_beg[xcd + 1];
     r.stride = per;
-    r.tail = r.cut > 1 && j < 4 * rem ? r.end + (j >> 2) : -1;
-    r.piece = j & 3;
+    if constexpr (CUT) {
+      const int round = __builtin_amdgcn_readfirstlane(lane_beg[xcd]) + per;
+      const int rem = __builtin_amdgcn_readfirstlane(r.end) - round;  // of the second round
+      if (p.hidden >= kCutK && rem > 0 && 4 * rem <= per && p.eto[p.E] <= kCutRows * p.E) {
+        r.end = round;
+        if (j < 4 * rem) r.tail = round + (j >> 2);
+        r.piece = j & 3;
+      }
+    }
   }
   return r;
 }
@@ -503,6 +514,7 @@ struct Gemm {
   static constexpr int WGM = Cfg<V>::WGM, WGN = Cfg<V>::WGN;
   static_assert(WGM * WGN == kConsumers, "one consumer wave per wave-grid cell");
   static constexpr int BK = Cfg<V>::BK, kStages = Cfg<V>::STAGES;
+  static constexpr bool kCut = V == UP_FWD;
   static constexpr int WM = BM / WGM, WN = BN / WGN;  // wave tile
   static constexpr int FM = WM / 32, FN = WN / 32;    // 32x32 blocks per wave
   static constexpr int A_STAGE = BM * BK * 2, B_STAGE = BN * BK * 2;  // bytes
@@ -953,9 +965,9 @@ struct Gemm {
   // expert with a wave-wide search of the prefix table from the cursor, then
   // its tile (for contig, that of lane slot `slot`) and K chunk. Every field
   // is workgroup-uniform.
-  // piece of cut: the item's share of the tile's columns (see Range).
+  // piece: the quarter of the tile's columns that is the item (see Range), -1: all.
   __device__ static Work decode(const Args& p, const Meta& mt, int item, int& ecur, int slot,
-                                int piece = 0, int cut = 1) {
+                                int piece) {
     const int lane = threadIdx.x & 63;
     int e = ecur;
     for (;;) {
@@ -996,8 +1008,8 @@ struct Gemm {
     w.m0 = mt_idx * BM;
     w.n0 = (tile - mt_idx * n_tiles) * BNO;
     w.nend = w.q.N;
-    if (!Cfg<V>::contig && cut > 1) {
-      const int cols = BNO / 4;
+    if (kCut && piece >= 0) {
+      constexpr int cols = BNO / 4;
       w.n0 += piece * cols;
       w.nend = min(w.q.N, w.n0 + cols);
       w.skip |= w.n0 >= w.q.N;
@@ -1472,7 +1484,7 @@ struct Gemm {
   // its slot, so the sum does not depend on which wave arrives last. Returns
   // true for that wave: acc then holds the whole tile for the normal
   // epilogue. No wave waits for another.
-  __device__ static bool split_arrive(const Args& p, const Meta& mt, const Range& rg, int a,
+  __device__ static bool split_arrive(const Args& p, const Meta& mt, const Range<kCut>& rg, int a,
                                       int chunks, int seg_item, f32x16_t (&acc)[FM][FN]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int NL = p.grid >> p.lsh, me = rg.lin >> p.lsh, ts = rg.slot;
@@ -1527,7 +1539,7 @@ struct Gemm {
   // (an item of fewer stages than the ring is deep, or the first one)
   // waits for its window explicitly.
   __device__ static void run_producer(const Args& p, lds_char* ring, lds_char* wins,
-                                      lds_char* scl, const Meta& mt, const Range& rg) {
+                                      lds_char* scl, const Meta& mt, const Range<kCut>& rg) {
     // The producer wave of each SIMD issues ahead of its two consumer waves
     // when both have an instruction ready: the DMAs are the stage's long pole
     // (s_setprio orders issue only; results do not change).
@@ -1589,7 +1601,7 @@ struct Gemm {
       if (!mapped) return;
       la_item = -1;
       for (int nx = rg.next(witem); nx >= 0; nx = rg.next(nx)) {
-        wla = decode(p, mt, nx, ela, rg.slot, rg.piece, rg.cut_of(nx));
+        wla = decode(p, mt, nx, ela, rg.slot, rg.piece_of(nx));
         if (wla.nk > 0) {
           TMap tn = tm;
           setup_map(p, wla, tn);
@@ -1606,7 +1618,7 @@ struct Gemm {
       while (inext >= 0) {
         witem = inext;
         wi = inext == la_item ? wla
-                              : decode(p, mt, inext, ei, rg.slot, rg.piece, rg.cut_of(inext));
+                              : decode(p, mt, inext, ei, rg.slot, rg.piece_of(inext));
         inext = rg.next(inext);
         if (wi.nk > 0) {
           ikt = 0;
@@ -1663,7 +1675,7 @@ struct Gemm {
   // end inside a split tile; such a segment is a partial sum, and the wave
   // that completes the tile's last segment stores the tile (split_arrive).
   __device__ static void run_consumer(const Args& p, const lds_char* ring, const Meta& mt,
-                                      const Range& rg, int total, lds_char* scr,
+                                      const Range<kCut>& rg, int total, lds_char* scr,
                                       const lds_char* scl) {
     int ec = 0;
     int s = 0;
@@ -1678,7 +1690,7 @@ struct Gemm {
     // Units flush kLead k-steps after their PRE loads are issued.
     constexpr int kLead = V == DOWN_DH ? 2 : 0;
     for (int item = rg.first(); item >= 0; item = rg.next(item)) {
-      const Work w = decode(p, mt, item, ec, rg.slot, rg.piece, rg.cut_of(item));
+      const Work w = decode(p, mt, item, ec, rg.slot, rg.piece_of(item));
       if (w.skip) continue;
       int slot = 0;
       if constexpr (kScaled) {
@@ -1763,7 +1775,7 @@ struct Gemm {
                              lds_char* wins, lds_char* scl) {
     const int total = build_meta(p, mt, (long long*)(char*)ring,
                                  (__attribute__((address_space(3))) int*)(ring + 256));
-    const Range rg = item_range<Cfg<V>::contig>(p, total, mt.lane_beg);
+    const Range<kCut> rg = item_range<Cfg<V>::contig, kCut>(p, total, mt.lane_beg);
     if (rg.first() < 0) return;
     const int wave = threadIdx.x >> 6;
     if (wave >= kConsumers)

@@ -454,9 +454,9 @@ extern "C" int vmoe_moe_forward(const uint16_t* logits, int64_t num_tokens, int3
     VMOE_TRY(vmoe_router_topk(logits, E, num_tokens, E, top_k, normalize, wts, sel, nullptr,
                               nullptr, lse, partial, nfl, nullptr, stream));
   }
-  // The losses ride in the routing launch where it takes them (one of the
-  // placement kernels that count for themselves, E <= 1024),
-  // else they get their own launch after the expert path.
+  // The losses ride in the routing launch where the top-k launch counts for it
+  // (route_hist_split: E a multiple of 8 up to 128, k a power of two up to 8);
+  // elsewhere they get their own launch after the expert path.
   const RouteAux aux = {partial, (int)M.partial_rows, num_tokens, coef, widths_normalized,
                         f_i, at<float>(saved, M.slot[VMOE_M_F_I32]),
                         at<float>(scratch, M.f_p_i), z_loss, losses};
@@ -570,10 +570,11 @@ extern "C" int vmoe_moe_backward(
     int32_t weight_grad, uint16_t* grad_x, int64_t ldgx, uint16_t* grad_w1, int64_t ldgw1,
     uint16_t* grad_w2, int64_t ldgw2, uint16_t* grad_logits, void* scratch, void* dw_workspace,
     size_t dw_workspace_bytes, vmoe_stream_t stream, vmoe_stream_t side_stream) {
-  return moe_backward(saved, logits, num_tokens, num_experts, top_k, normalize, block_size, x, ldx, w1, ldw1, w2,
-      ldw2, ewo, widths, hidden, max_width, coef, widths_normalized, grad_out, ldg, grad_scale, grad_z,
-      grad_lb, grad_cl, weight_grad, grad_x, ldgx, grad_w1, ldgw1, grad_w2, ldgw2, grad_logits,
-      scratch, dw_workspace, dw_workspace_bytes, stream, side_stream, nullptr);
+  return moe_backward(saved, logits, num_tokens, num_experts, top_k, normalize, block_size, x, ldx,
+                      w1, ldw1, w2, ldw2, ewo, widths, hidden, max_width, coef, widths_normalized,
+                      grad_out, ldg, grad_scale, grad_z, grad_lb, grad_cl, weight_grad, grad_x,
+                      ldgx, grad_w1, ldgw1, grad_w2, ldgw2, grad_logits, scratch, dw_workspace,
+                      dw_workspace_bytes, stream, side_stream, nullptr);
 }
 
 extern "C" int vmoe_moe_router_backward(
@@ -590,8 +591,9 @@ extern "C" int vmoe_moe_router_backward(
     void* router_workspace, size_t router_workspace_bytes) {
   const RouterGrad router = {wr, ldwr, grad_wr, ldgwr, need_x != 0, router_workspace,
                              router_workspace_bytes};
-  return moe_backward(saved, logits, num_tokens, num_experts, top_k, normalize, block_size, x, ldx, w1, ldw1, w2,
-      ldw2, ewo, widths, hidden, max_width, coef, widths_normalized, grad_out, ldg, grad_scale, grad_z,
-      grad_lb, grad_cl, weight_grad, grad_x, ldgx, grad_w1, ldgw1, grad_w2, ldgw2, grad_logits,
-      scratch, dw_workspace, dw_workspace_bytes, stream, side_stream, &router);
+  return moe_backward(saved, logits, num_tokens, num_experts, top_k, normalize, block_size, x, ldx,
+                      w1, ldw1, w2, ldw2, ewo, widths, hidden, max_width, coef, widths_normalized,
+                      grad_out, ldg, grad_scale, grad_z, grad_lb, grad_cl, weight_grad, grad_x,
+                      ldgx, grad_w1, ldgw1, grad_w2, ldgw2, grad_logits, scratch, dw_workspace,
+                      dw_workspace_bytes, stream, side_stream, &router);
 }

@@ -282,9 +282,9 @@ __device__ __forceinline__ void mfma4(f32x16_t& acc, const float4& a, const floa
   acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
 }
 
-// The expert and tile of item j of this workgroup's XCD: each wave counts the tiles of 64
-// experts at a time, one per lane, and scans them (a walk over the experts one
-// by one costs a dependent load per expert). XCD x takes a contiguous eighth
+// The expert and tile of item j of this workgroup's XCD: each wave counts the
+// tiles of 64 experts at a time, one per lane, and scans them (a walk over the
+// experts one by one costs a dependent load per expert). XCD x takes a contiguous eighth
 // of the tiles, so the tiles that share rows or columns share an L2. Returns
 // false past the last tile.
 template <int F>

@@ -276,11 +276,15 @@ inline bool span_ok(int64_t rows, int64_t ld) { return rows * ld * 2 < ((int64_t
 // A workgroup here does one tile, started cold, and ends, where the persistent
 // 128 x 256 kernel loads its next tile during the last one's k-steps. So these
 // win while one round of the 256 CUs, or a little more, takes all tiles. Whole
-// forward in a graph, us with 128 x 256 tiles and with these: 8 experts 768 -> 512 at 24 row blocks (192 + 288 tiles) 47.8 and 34.1,
-// at 40 (up 320 of these, down 480 of the old) 49.7 and 47.4; 64 experts 1024 ->
-// 256 at 72 - 96 blocks (up 288 - 384) 56.7 and 48.9, 58.9 and 50.2. Without the
-// line: 64 experts at 128 blocks (512 and 2048 tiles) 61.8 and 61.6, at 192 69.5
-// and 79.6; 128 experts 2048 -> 1024 / 512 / 256 185 and 258.
+// forward in a graph, us with 128 x 256 tiles and with these: 8 experts 768 ->
+// 512 at 24 row blocks (192 + 288 tiles) 47.8 and 34.1, at 40 (up 320 of these,
+// down 480 of the old) 49.7 and 47.4; 64 experts 1024 -> 256 at 72 - 96 blocks
+// (up 288 - 384) 56.7 and 48.9, 58.9 and 50.2. Without the line: 64 experts at
+// 128 blocks (512 and 2048 tiles) 61.8 and 61.6, at 192 69.5 and 79.6; 128
+// experts 2048 -> 1024 / 512 / 256 185 and 258. With it, 140 forwards drawn over
+// 1-128 experts, widths 64-1024, 64-2048 hidden columns and 1-512 tokens are
+// 0.98-1.4 times as fast as without, 1.20 in the mean (below 1 where neither
+// projection takes these tiles).
 bool few_rows_fits(int64_t assignments, int64_t E, int64_t cols) {
   return cols > 0 && live_blocks(assignments, E) * ((cols + kTile - 1) / kTile) <= kFewRowsItems;
 }

@@ -1,9 +1,10 @@
 // The router's auxiliary-loss reduction as the device code of one 1024-thread
 // workgroup. router_aux_kernel (router.hip) runs it as a launch of its own;
-// route_small_kernel and route_fused_kernel (route.hip) run it in one extra workgroup beside the
-// routing placement when the MoE layer asks for it, so the layer's forward
-// has one launch fewer. Both run the same code with the same thread mapping,
-// so the losses carry the same bits either way.
+// route_small_kernel and route_fused_kernel (route.hip) run it in one extra
+// workgroup beside the routing placement when the MoE layer asks for it (where
+// its top-k launch counts for the routing), so the layer's forward has one
+// launch fewer. Both run the same code with the same thread mapping, so the
+// losses carry the same bits either way.
 #pragma once
 
 #include "vmoe_common.h"

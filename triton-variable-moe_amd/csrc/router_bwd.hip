@@ -212,7 +212,11 @@ __device__ __forceinline__ void rb_combine(const RbArgs& p, const int32_t (&idx)
 // back (combine and this launch, then this launch alone: 52 + 29 -> 74 us at
 // 16384 x 1024, E = 64, k = 8; 15 + 19 -> 23 us at 16384 x 768, E = 16, k = 2).
 // Up to 64 experts: at 128 the larger tile of w leaves fewer workgroups per CU
-// for the row reads (32768 x 2048, k = 8: 213 + 107 against 323 us).
+// for the row reads (32768 x 2048, k = 8: 213 + 107 against 323 us). Between
+// them it depends on the slots and the tokens: training steps of 72 and 96
+// experts, 512-2048 wide, took with the sum here 0.96-1.00 of their time at
+// k = 2, 0.97-1.01 at k = 8 from 4096 tokens and up to 1.04 at 1024 tokens (the
+// launch's few workgroups each wait for 8 rows a token), so the line stays.
 template <int MB, int KMAX>
 __device__ __forceinline__ void rb_grad_x(const RbArgs& p, int block, char* lds) {
   rb_lds* ws = (rb_lds*)lds;
@@ -355,7 +359,8 @@ __global__ __launch_bounds__(256) void router_linear_sum_kernel(const float* __r
       make_uint2(pack_bf16(s.x, s.y), pack_bf16(s.z, s.w));
 }
 
-// About one grad_w workgroup per CU (256), at least one stage of tokens each.
+// About one grad_w workgroup per CU of a whole MI355X (256; a part of one runs
+// them in turn), at least one stage of tokens each.
 void rb_split(int64_t T, int64_t d, int& slabs, int& chunks, int& per) {
   slabs = (int)((d + kRbCols - 1) / kRbCols);
   const int64_t stages = (T + kRbTokens - 1) / kRbTokens;

@@ -752,13 +752,14 @@ def test_column_slice_operands(device):
         assert bits_equal(a, b)
 
 
-@pytest.mark.parametrize("K,rows", [(1536, 8), (1544, 8), (1528, 8), (1544, 168)])
-def test_cut_last_round_same_bits(K, rows, device):
-    """280 or 288 tiles: from 1536 hidden columns and up to 160 rows an
-    expert, one round of 256 CUs and 24 tiles cut into column pieces (the widths
-    end inside a piece), give the bits of the same experts in two calls, which
-    cut none; as do the shapes that lie just past either line."""
-    E, w = (70, 1000) if rows == 8 else (36, 1000)
+@pytest.mark.parametrize("E,w,K,rows", [
+    (70, 1000, 1024, 8), (70, 1000, 1032, 8),     # cut; the widths end inside a piece
+    (70, 1000, 1016, 8), (36, 1000, 1032, 168),   # K, or several row tiles: not
+    (70, 200, 1032, 392), (40, 200, 1032, 776)])  # one column tile: up to 768 rows
+def test_cut_last_round_same_bits(E, w, K, rows, device):
+    """280 or 288 tiles, one round of 256 CUs and a last one that is cut into
+    column pieces, or just past a line of that rule, give the bits of the same
+    experts in two calls, which cut none."""
     g = torch.Generator().manual_seed(11)
     x = torch.randn(E * rows, K, generator=g).to(torch.bfloat16).to(device)
     w1 = (torch.randn(K, E * w, generator=g) * 0.05).to(torch.bfloat16).to(device)

@@ -112,6 +112,7 @@ struct Args {
   int paired;        // 1: one of the two GEMMs of grouped_gemm_pair_kernel (see vblock)
   float* row_dot;    // DOWN_DH with pre: per (row, 64-column block) sum of GH * PRE^2 (nullable)
   int64_t ld_rd;     // its leading dimension (floats)
+  int64_t cut_rows;  // UP_FWD: padded rows per expert up to which a last round is cut (Range)
 };
 
 // Metadata of one expert as the GEMMs read it: its row range [t0, t1) in
@@ -438,16 +439,18 @@ struct Range {
   // quarter of another, the tiles of that second round are cut along n into
   // four pieces, so that four times as many workgroups share it; this workgroup
   // takes piece `piece` of tile `tail` (-1: none). A piece takes as many
-  // k-steps and staging instructions as its tile and a quarter of the bytes of
-  // B, so it pays where the tail waits for weights: K at least kCutK, and few
-  // rows per expert (kCutRows). Forwards of 60 layers drawn with 260-310 tiles
-  // and 20-105 rows an expert, without / with the cut: 1.00-1.05 (mean 1.02)
-  // at K = 2048-4096, 0.99-1.04 at 1536, 0.98-1.02 at 1024; with 150-500 rows
-  // an expert at K = 1536-2048 0.97-1.01. 1531 tokens through 128 experts of
-  // 256-1024, K = 2048: the up projection 104 -> 89 us, the layer 226 -> 214.
+  // k-steps, staging instructions and MFMAs of a wave as its tile and a quarter
+  // of the bytes of B, so it pays where the tail waits for weights (cut_rows).
+  // Forwards without / with the cut, weights not in cache: 60 layers drawn with
+  // 260-310 tiles, 20-105 rows an expert and K = 1024-4096 1.00-1.05 (mean
+  // 1.02); K = 512-768 0.98-1.01; several row tiles an expert and several
+  // column tiles 0.97-1.03 (mean 0.995); one column tile, up to 768 rows 0.995-
+  // 1.027 (mean 1.005), more rows 0.98-1.007 (0.998). 1531 tokens through 128
+  // experts of 256-1024, K = 2048: the up projection 104 -> 89 us, the layer 226
+  // -> 214; 4101 x 8 rows through 64 experts of 256, K = 1024: 47.7 -> 44.0 us.
   // Not taken: more rounds, or a fuller last one in halves (up to 1 % slower),
-  // and no full round before it (64 tokens, 64 experts of 256: 20.3 -> 22.0
-  // us). The other forms gained nothing (the code spilled scalars in dH).
+  // no full round before it (64 tokens, 64 experts of 256: 20.3 -> 22.0 us), the
+  // other forms (no gain; the code spilled scalars in dH).
   int tail, piece;
   // The workgroup's items in order: beg, beg + stride, ... below end, then the
   // tail; -1 past the last.
@@ -461,7 +464,12 @@ struct Range {
     return CUT && item >= end ? piece : -1;
   }
 };
-constexpr int kCutK = 1536, kCutRows = 160;  // kCutRows: padded rows per expert
+// Padded rows per expert up to which the up projection's last round is cut: one
+// row tile and a little, or six where an expert is one column tile wide (more
+// column tiles multiply the workgroups that read the same token rows at once).
+inline int64_t cut_rows(int64_t hidden, int64_t max_width) {
+  return hidden < 1024 ? 0 : max_width <= 256 ? 768 : 160;
+}
 
 // The workgroup's index among the p.grid workgroups of its GEMM. A paired
 // launch (grouped_gemm_pair_kernel) deals consecutive groups of 8 workgroups
@@ -497,7 +505,7 @@ __device__ __forceinline__ Range<CUT> item_range(const Args& p, int total, const
     if constexpr (CUT) {
       const int round = __builtin_amdgcn_readfirstlane(lane_beg[xcd]) + per;
       const int rem = __builtin_amdgcn_readfirstlane(r.end) - round;  // of the second round
-      if (p.hidden >= kCutK && rem > 0 && 4 * rem <= per && p.eto[p.E] <= kCutRows * p.E) {
+      if (rem > 0 && 4 * rem <= per && p.eto[p.E] <= p.cut_rows * p.E) {
         r.end = round;
         if (j < 4 * rem) r.tail = round + (j >> 2);
         r.piece = j & 3;
@@ -2181,6 +2189,7 @@ extern "C" int vmoe_gemm_up_fwd(const uint16_t* x, int64_t ldx, int64_t x_rows,
   p.b = w1; p.ldb = ldw1;
   p.c = out; p.c2 = activation == VMOE_ACT_RELU_SQUARED ? pre_act : nullptr; p.ldc = ldo;
   p.row_scale = row_scale;
+  p.cut_rows = cut_rows(hidden, max_width);
   p.eto = eto; p.ewo = ewo; p.widths = widths; p.tpe = tpe;
   p.E = E; p.hidden = (int)hidden; p.act = activation; p.rows_bound = rows_bound;
   return launch<UP_FWD>(p, row_items<UP_FWD>(rows_bound, E, max_width),

@@ -1306,7 +1306,9 @@ def _moe_backward(ctx, grad_out, g_z, g_lb, g_cl, need_logits, need_experts, rou
 
 def _scalar_f32(g):
     """A loss gradient as the device fp32 scalar the kernels read (None: none)."""
-    return None if g is None else g.detach().to(torch.float32).reshape(()).contiguous()
+    if g is None or (g.dtype == torch.float32 and g.dim() == 0):
+        return g  # only its address is read
+    return g.detach().to(torch.float32).reshape(()).contiguous()
 
 
 _MOE_F32_PLANS: dict[tuple, tuple] = {}
